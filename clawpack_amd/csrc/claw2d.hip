@@ -37,7 +37,7 @@ namespace claw {
 
 constexpr int kLanes = 64;
 constexpr int kOwn = 60;  // owned columns per strip
-constexpr int kWPB = 4;   // independent wavefronts per workgroup
+constexpr int kWPB = 4;   // independent wavefronts per workgroup, at least
 // Shallow-water steady rows per segment from which issue priority follows progress (shorter
 // segments ran 0.5-2% slower with it on MI355X: 2048^2 and below)
 constexpr int kPrioRows = 64;
@@ -182,7 +182,7 @@ template <class T, class P> struct StepArgs {
   int abx_lo, abx_hi, aby_lo, aby_hi;
   // the capacity plane kappa (aux plane mcapa-1) of a capacity-form step, else null
   const T* capa;
-  // launch shape: wavefronts per workgroup (1, 2 or 4) and XCD-contiguous order (1) or not (0)
+  // launch shape: wavefronts per workgroup and XCD-contiguous order (1) or not (0)
   int wpb, xcd;
   typename P::Par par;
 };
@@ -326,10 +326,24 @@ __device__ __forceinline__ double uniform(double v) {
 }
 
 // Folds maxima into a control block (every lane issues the atomics with the same operand, so the
-// call may sit in wave-uniform control flow inside a work loop).
-__device__ __forceinline__ void publish_max(claw2d_ctrl* c, const ItemMax& m) {
-  atomic_max_nonneg(&c->smax_bits[0], m.sx);
-  atomic_max_nonneg(&c->smax_bits[1], m.sy);
+// call may sit in wave-uniform control flow inside a work loop).  `many`: the maxima are looked up
+// first and an atomic is sent only for one that would rise.  Device-scope atomics on one line
+// are served one after another, and a launch's workgroups finish close together, so with many of
+// them the queue shows (Euler FP32 1501 x 1207, 452 workgroups: 56.3 -> 50.9 us; shallow water
+// 1024^2, 234: 45.4 -> 43.3 us); with few the extra round trip costs more (64^2, 8: 18.8 -> 19.3
+// us; 512^2, 126: no change).  The lookup is a device-scope atomic load, and a maximum only rises
+// during a step, so a maximum that is left out was already covered.
+constexpr int kManyGroups = 128;
+__device__ __forceinline__ void publish_max(claw2d_ctrl* c, const ItemMax& m, bool many) {
+  const double sx = many ? uniform(__longlong_as_double((long long)__hip_atomic_load(
+                               &c->smax_bits[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)))
+                         : 0.0;
+  const double sy = many ? uniform(__longlong_as_double((long long)__hip_atomic_load(
+                               &c->smax_bits[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)))
+                         : 0.0;
+  // compared as the atomics compare them (bit patterns of non-negative doubles; a NaN is the largest)
+  if (!many || __double_as_longlong(m.sx) > __double_as_longlong(sx)) atomic_max_nonneg(&c->smax_bits[0], m.sx);
+  if (!many || __double_as_longlong(m.sy) > __double_as_longlong(sy)) atomic_max_nonneg(&c->smax_bits[1], m.sy);
   if (m.bad) atomicOr(&c->status, (int)CLAW_STATUS_BAD_STATE);
 }
 
@@ -826,12 +840,20 @@ __device__ __forceinline__ void control_one(claw2d_ctrl* c, double dx, double dy
 #ifndef CLAW_MIN_WAVES_F32
 #define CLAW_MIN_WAVES_F32 0
 #endif
+// Wavefronts per workgroup a single-grid kernel is built for: those one CU holds at the kernel's
+// registers (FP64 2 per SIMD, its specialised split kernels 3; FP32 4, Euler 3), so that a CU can
+// run one workgroup, which sends one set of atomics.  FP64 Euler keeps 4: 8 gained nothing there.
+// METHOD: the method is fixed at compile time.
+template <class T, class P, bool SPLIT, bool METHOD>
+constexpr int kMaxWPB =
+    sizeof(T) == 8 ? (P::NEQ == 4 ? 4 : (SPLIT && METHOD ? 12 : 8)) : (P::NEQ == 3 ? 16 : 12);
+
 template <class T> struct MinWaves {
   static constexpr int value = sizeof(T) == 8 ? CLAW_MIN_WAVES_F64 : CLAW_MIN_WAVES_F32;
 };
 
 template <class T, class P, int LIM, bool SPLIT, int TWC, bool PAD = false, int SWEEP = 0, bool CAPA = false>
-__global__ void __launch_bounds__(kLanes* kWPB) __attribute__((amdgpu_waves_per_eu(MinWaves<T>::value)))
+__global__ void __launch_bounds__(kLanes*(kMaxWPB<T, P, SPLIT, (LIM > 0)>)) __attribute__((amdgpu_waves_per_eu(MinWaves<T>::value)))
 step2_fused(StepArgs<T, P> a) {
   // The wavefronts of a workgroup combine their speed maxima and bad-state flags in LDS; the last
   // of them to finish folds the workgroup's into the control block and counts the workgroup in
@@ -878,7 +900,7 @@ step2_fused(StepArgs<T, P> a) {
       uniform(__longlong_as_double(
           (long long)__hip_atomic_load(&wg_smax[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP))),
       __builtin_amdgcn_readfirstlane(__hip_atomic_load(&wg_bad, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP)) != 0};
-  publish_max(a.ctrl, wg);
+  publish_max(a.ctrl, wg, gridDim.x >= kManyGroups);
   if (a.fuse) {
     // The last workgroup to finish closes the step: the speed maxima are then complete.  The wait
     // for this wavefront's outstanding memory operations (its max/or atomics are acknowledged once
@@ -936,7 +958,7 @@ batch_step(StepArgs<T, P> a, BatchDev b) {
     const int strip = local % G.nstrips, seg = local / G.nstrips;
     const int x0 = strip * kOwn, y0 = seg * G.seg_h;
     const int y1 = min(y0 + G.seg_h, G.my);
-    publish_max(c, march_item<T, P, LIM, false, TWC>(a, qin, qout, G.mx, G.my, x0, y0, y1, dt, G.dx, G.dy));
+    publish_max(c, march_item<T, P, LIM, false, TWC>(a, qin, qout, G.mx, G.my, x0, y0, y1, dt, G.dx, G.dy), false);
   }
 }
 
@@ -1040,11 +1062,6 @@ static long resident_waves(const void* kern, int wpb = kWPB) {
   return (long)cus * std::min<long>((long)bpc * wpb, kMaxWavesPerCU);
 }
 
-// wavefronts per workgroup of a single-grid launch (desc->wg_waves; 0 = kWPB)
-static int launch_wpb(const claw2d_desc* d) { return d->wg_waves > 0 ? d->wg_waves : kWPB; }
-// occupancy cache index of a wavefronts-per-workgroup count 1, 2 or 4
-static int wpb_index(int wpb) { return wpb == 1 ? 0 : (wpb == 2 ? 1 : 2); }
-
 // SIMDs of the current device (4 per CU), 0 if the query fails.
 static long device_simds() {
   static thread_local long simds = -1;
@@ -1056,6 +1073,21 @@ static long device_simds() {
   }
   return simds;
 }
+
+// wavefronts per workgroup of a single-grid launch (desc->wg_waves; 0 = kWPB)
+static int launch_wpb(const claw2d_desc* d) { return d->wg_waves > 0 ? d->wg_waves : kWPB; }
+// The default packing of a launch of `items` wavefronts: 4 per workgroup (one per SIMD) while that
+// leaves at most one workgroup per CU, else as many as spread the wavefronts evenly over the CUs
+// in one workgroup each, up to what the kernel is built for.  Fewer, larger workgroups send fewer
+// atomics (beside the lookup in publish_max: shallow water 2048^2 FP32 70.8 -> 69.2 us, bathymetry
+// FP32 69.9 -> 66.2 us, FP64 minmod 97.3 -> 94.8 us).
+static int fit_wpb(const claw2d_desc* d, long items, int most) {
+  const long cus = device_simds() / 4;
+  if (launch_wpb(d) < kWPB || cus <= 0) return launch_wpb(d);
+  return (int)std::min<long>(most, std::max<long>(kWPB, (items + cus - 1) / cus));
+}
+// occupancy cache index of a wavefronts-per-workgroup count 1, 2 or 4
+static int wpb_index(int wpb) { return wpb == 1 ? 0 : (wpb == 2 ? 1 : 2); }
 
 // Rows per marching segment.  A wavefront's run time is proportional to its rows, so the grid
 // is cut into as many segments as fit in one resident round (every wavefront starts at once
@@ -1238,11 +1270,10 @@ static int launch_step(const claw2d_desc* d, const typename P::Par& par, void* q
   } else if (!pad || SPLIT) {
     kern = step_kernel<T, P, SPLIT>(d, &slot);
   }
-  const int wpb = launch_wpb(d);
   static thread_local long cached[7][3] = {{-1, -1, -1}, {-1, -1, -1}, {-1, -1, -1}, {-1, -1, -1},
                                            {-1, -1, -1}, {-1, -1, -1}, {-1, -1, -1}};
-  long& res = cached[slot][wpb_index(wpb)];
-  if (res < 0) res = resident_waves(kern, wpb);
+  long& res = cached[slot][wpb_index(launch_wpb(d))];
+  if (res < 0) res = resident_waves(kern, launch_wpb(d));
   StepArgs<T, P> a;
   fill_args(a, d, res);
   a.q0 = (T*)q0;
@@ -1260,6 +1291,8 @@ static int launch_step(const claw2d_desc* d, const typename P::Par& par, void* q
   if (d->mcapa > 0) a.capa = (const T*)aux + (size_t)(d->mcapa - 1) * (size_t)d->mx * (size_t)d->my;
   const int waves = a.nstrips * a.nsegs;
   a.total_waves = waves;
+  const int wpb = a.wpb =
+      fit_wpb(d, waves, SPLIT && slot < 2 ? kMaxWPB<T, P, SPLIT, true> : kMaxWPB<T, P, SPLIT, false>);
   const int blocks = (waves + wpb - 1) / wpb;
   void* args[] = {&a};
   const hipError_t e = hipLaunchKernel(kern, dim3(blocks), dim3(kLanes * wpb), args, 0, s);

@@ -96,7 +96,8 @@ typedef struct claw2d_desc {
    * take only 0.  claw2d_mass_sum returns the sum of h (depth_ref times the cell count added). */
   double depth_ref;
   /* Launch shape of the single-grid step kernels (results do not depend on it): wavefronts per
-   * workgroup, 1, 2 or 4 (0 = 4), and the order in which workgroups take strips and segments,
+   * workgroup, 1, 2 or 4 (0 = 4; with 4 the library packs more where that fills the CUs evenly),
+   * and the order in which workgroups take strips and segments,
    * 0 = each XCD takes a contiguous range (neighbouring strips share halo lines in one L2),
    * 1 = plain order (workgroup b to the XCD b mod 8, as dispatched). */
   int32_t wg_waves;
