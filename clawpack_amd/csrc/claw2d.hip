@@ -216,7 +216,7 @@ __device__ __forceinline__ typename P::Cell prep_cell(const T q[P::NEQ], T b, co
 // (dt/dx)(1/kappa_L + 1/kappa_R)/2 in place of dt/dx, and the transverse terms of amdq (apdq)
 // carry dt/(dx kappa) of the left (right) cell.
 template <class T, class P, int LIM, int TWC, bool CAPA = false>
-__device__ __forceinline__ void finish_iface(const typename P::Iface& f, const T upL[P::NW],
+__device__ __forceinline__ void finish_iface(const typename P::Iface& f, const T sfs[P::NW], const T upL[P::NW],
                                              const T alR[P::NW], const T mR[P::NW], T r, T rt,
                                              const StepArgs<T, P>& a, T LX[P::NEQ], T LG1[P::NEQ],
                                              T LG2[P::NEQ], T RX[P::NEQ], T RG1[P::NEQ],
@@ -231,7 +231,7 @@ __device__ __forceinline__ void finish_iface(const typename P::Iface& f, const T
   T XL[NW], XR[NW], A[NW], B[NW];
 #pragma unroll
   for (int p = 0; p < NW; ++p) {
-    const T s = P::speed(f, p), al = f.al[p], sf = f.sf[p];
+    const T s = P::speed(f, p), al = f.al[p], sf = sfs[p];
     const T e = sf * al, q = P::FWAVE ? al - e : (s - sf) * al;
     T k = T(0);
     if (second) {
@@ -270,12 +270,12 @@ __device__ __forceinline__ void finish_iface(const typename P::Iface& f, const T
       P::tspeeds(f, tc, sg);
 #pragma unroll
       for (int j = 0; j < NW; ++j) {
-        const T wm = wA * vmin(sg[j], T(0)), wp = wA * vmax(sg[j], T(0));
+        const T wm = wA * vmin0(sg[j]), wp = wA * vmax0(sg[j]);
         c1[j] = wm * bA[j];
         c2[j] = wp * bA[j];
         if constexpr (CAPA) {
-          c3[j] = (wB * vmin(sg[j], T(0))) * bB[j];
-          c4[j] = (wB * vmax(sg[j], T(0))) * bB[j];
+          c3[j] = (wB * vmin0(sg[j])) * bB[j];
+          c4[j] = (wB * vmax0(sg[j])) * bB[j];
         } else {
           c3[j] = wm * bB[j];
           c4[j] = wp * bB[j];
@@ -286,6 +286,77 @@ __device__ __forceinline__ void finish_iface(const typename P::Iface& f, const T
       P::expand_t(f, tc, c3, RG1);
       P::expand_t(f, tc, c4, RG2);
     }
+  }
+}
+
+// finish_iface of a plain interface (P::plain), the same bit for bit: wave p of side -1 is
+// left-going (sf = s, no right-going part, the limiter's partner is the right interface), of side
+// 1 right-going, of side 0 either; the transverse split has its fixed pattern.  Parts that
+// finish_iface multiplies by zero or adds to zero are left out.
+template <class T, class P, int LIM, int TWC, bool CAPA = false>
+__device__ __forceinline__ void finish_plain(const typename P::Iface& f, const T upL[P::NW], const T alR[P::NW],
+                                             const T mR[P::NW], T r, T rt, const StepArgs<T, P>& a, T LX[P::NEQ],
+                                             T LG1[P::NEQ], T LG2[P::NEQ], T RX[P::NEQ], T RG1[P::NEQ],
+                                             T RG2[P::NEQ], T rkL = T(1), T rkR = T(1)) {
+  constexpr int NEQ = P::NEQ, NW = P::NW;
+  const bool second = TWC >= 0 ? true : a.order != 1;
+  const int tw = TWC >= 0 ? TWC : a.tw;
+  const bool fold = second && tw == 2;
+  T in[NW];
+  if (second) P::inv_norm(f, in);
+  const T rc = CAPA ? T(0.5) * (r * rkL + r * rkR) : r;
+  T XL[NW], XR[NW], A[NW], B[NW];
+#pragma unroll
+  for (int p = 0; p < NW; ++p) {
+    const int side = P::side(p);
+    const T s = P::speed(f, p), al = f.al[p];
+    T k = T(0);
+    if (second) {
+      const T aR = alR[p], mr = mR[p];
+      T t;
+      if (side < 0) t = (aR * mr) * in[p];
+      else if (side > 0) t = upL[p] * in[p];
+      else t = (s > T(0) ? upL[p] : aR * mr) * in[p];
+      const int meth = LIM > 0 ? LIM : a.mthlim[p];
+      const T sa = side < 0 ? -s : (side > 0 ? s : vabs(s));
+      const T sw = P::FWAVE ? (side < 0 ? T(-1) : (side > 0 ? T(1) : copysign(T(1), s))) : sa;
+      k = sw * (T(1) - sa * rc) * limited(al, t, meth);
+    }
+    const T hk = T(0.5) * k;
+    if (side < 0) {
+      const T e = P::FWAVE ? al : s * al;
+      XL[p] = -r * fma(T(0.5), k, e);
+      XR[p] = r * hk;
+      A[p] = fold ? e + k : e;
+      B[p] = fold ? -k : T(0);
+    } else if (side > 0) {
+      const T q = P::FWAVE ? al : s * al;
+      XL[p] = -r * hk;
+      XR[p] = -r * fma(T(-0.5), k, q);
+      A[p] = fold ? k : T(0);
+      B[p] = fold ? q - k : q;
+    } else {
+      const T sf = P::plain_fix(s);
+      const T e = sf * al, q = P::FWAVE ? al - e : (s - sf) * al;
+      XL[p] = -r * fma(T(0.5), k, e);
+      XR[p] = -r * fma(T(-0.5), k, q);
+      A[p] = fold ? e + k : e;
+      B[p] = fold ? q - k : q;
+    }
+  }
+  P::expand_n(f, XL, LX);
+  P::expand_n(f, XR, RX);
+#pragma unroll
+  for (int m = 0; m < NEQ; ++m) LG1[m] = LG2[m] = RG1[m] = RG2[m] = T(0);
+  if (tw > 0) {
+    T bA[NW], bB[NW];
+    P::tbeta(f, A, bA);
+    P::tbeta(f, B, bB);
+    const T w = T(-0.5) * r * rt;
+    const T wA = CAPA ? T(-0.5) * (r * rkL) * rt : w, wB = CAPA ? T(-0.5) * (r * rkR) * rt : w;
+    const typename P::TConst tc = P::tconst(f);
+    P::expand_t_split(f, tc, wA, bA, LG1, LG2);
+    P::expand_t_split(f, tc, wB, bB, RG1, RG2);
   }
 }
 
@@ -325,6 +396,14 @@ __device__ __forceinline__ double uniform(double v) {
   return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
 }
 
+// A wavefront-uniform pointer that the compiler keeps in scalar registers: it otherwise folds the
+// lane's column into it, and the row loop then adds the row to a 64-bit vector address per plane
+// (six vector additions per row) in place of one scalar addition.
+template <class T> __device__ __forceinline__ T* scalar_ptr(T* p) {
+  asm("" : "+s"(p));
+  return p;
+}
+
 // Folds maxima into a control block (every lane issues the atomics with the same operand, so the
 // call may sit in wave-uniform control flow inside a work loop).  `many`: the maxima are looked up
 // first and an atomic is sent only for one that would rise.  Device-scope atomics on one line
@@ -361,6 +440,11 @@ __device__ __forceinline__ ItemMax march_item(const StepArgs<T, P>& a, const T* 
   // the interfaces at lanes 2..62, whose inputs come from lanes 1..63 (measured on MI355X: FP64
   // shallow water -3.7% together with the one-way limiter exchange below, Euler FP32 -4%).
   constexpr bool DPPZ = true;
+  // lanes whose interfaces reach an owned cell (2..61): x-interfaces 2..62, and the y-interfaces of
+  // columns 1..62, or of the owned columns alone where nothing crosses columns (split)
+  constexpr unsigned long long kXLanes = 0x7ffffffffffffffcull;
+  constexpr unsigned long long kYLanes = SPLIT ? 0x3ffffffffffffffcull : 0x7ffffffffffffffeull;
+  constexpr bool TRANS = TWC != 0;  // interfaces are split transversely (possibly)
   constexpr int NEQ = P::NEQ, NW = P::NW, NC = P::NC, NL = P::NL;
   // 4 equations: add each y-interface's upper-cell shares at once (two more exchanges per row)
   // instead of carrying them to the next row, so the kernel fits 2 wavefronts per SIMD
@@ -380,50 +464,51 @@ __device__ __forceinline__ ItemMax march_item(const StepArgs<T, P>& a, const T* 
     map_index(c, mx, a.abx_lo, a.abx_hi, cxa, fa);
   }
   const bool own_col = lane >= 2 && lane < 2 + kOwn && c < mx;
-  const bool xcfl_col = lane >= 1 && c >= 0 && c <= mx;   // x-interfaces 1..mx+1 (1-based)
-  const bool ycfl_col = c >= -1 && c <= mx;               // y-sweeps on columns 0..mx+1
   const T dtdx = T(dt / dx), dtdy = T(dt / dy);
 
   // Loads row R of this lane's column.  The wall sign flips are returned, not applied, so the
   // consumer (one row later) and not the load waits for the data.
-  const bool walls = !PAD && (fx || a.bcy_lo == CLAW_BC_WALL || a.bcy_hi == CLAW_BC_WALL);
+  const bool xflips = __builtin_amdgcn_ballot_w64(fx) != 0ull;  // some column mirrors a wall
   const ptrdiff_t ldq = PAD ? (ptrdiff_t)mx + 4 : (ptrdiff_t)mx;  // row stride of qin
   const size_t plane_in = PAD ? (size_t)(mx + 4) * (size_t)(my + 4) : plane;
-  const T* const qin0 = PAD ? qin + 2 * ldq + 2 : qin;             // cell (0, 0)
-  auto load_row = [&](int R, T q[NEQ], bool& fy, T& b, T& kap, T& kapx) {
+  const T* const qin0 = PAD ? qin + 2 * ldq : qin;                 // row 0, and the lane's column in it
+  const unsigned qcol = (unsigned)(PAD ? cx + 2 : cx);
+  const bool fx0 = fx && a.rfx == 0, fx1 = fx && a.rfx == 1, fx2 = fx && a.rfx == 2, fx3 = fx && a.rfx == 3;
+  // IN: the row is in the grid (no ghost row), known at the call
+  auto load_row = [&](int R, T q[NEQ], bool& fy, T& b, T& kap, T& kapx, auto in_tag) {
+    constexpr bool IN = decltype(in_tag)::value;
     int ry = R;
     fy = false;
-    if constexpr (!PAD) {
+    if constexpr (!PAD && !IN) {
       if (R < 0 || R >= my) map_index(R, my, a.bcy_lo, a.bcy_hi, ry, fy);
     }
     ry = __builtin_amdgcn_readfirstlane(ry);
-    const T* src = qin0 + (ptrdiff_t)ry * ldq + (ptrdiff_t)cx;
+    // uniform row pointer + the lane's column as an unsigned offset: scalar address arithmetic
+    const T* src = qin0 + (ptrdiff_t)ry * ldq;
 #pragma unroll
-    for (int m = 0; m < NEQ; ++m) q[m] = src[(size_t)m * plane_in];
-    if constexpr (P::NAUX > 0) {
+    for (int m = 0; m < NEQ; ++m) q[m] = scalar_ptr(src + (size_t)m * plane_in)[qcol];
+    if constexpr (P::NAUX > 0 || CAPA) {
       int ra = R;
-      bool fa;
-      if (R < 0 || R >= my) map_index(R, my, a.aby_lo, a.aby_hi, ra, fa);
+      if constexpr (!IN) {
+        bool fa;
+        if (R < 0 || R >= my) map_index(R, my, a.aby_lo, a.aby_hi, ra, fa);
+      }
       ra = __builtin_amdgcn_readfirstlane(ra);
-      b = a.aux[(size_t)ra * (size_t)mx + (size_t)cxa];
-    }
-    if constexpr (CAPA) {
-      int ra = R;
-      bool fa;
-      if (R < 0 || R >= my) map_index(R, my, a.aby_lo, a.aby_hi, ra, fa);
-      ra = __builtin_amdgcn_readfirstlane(ra);
-      kap = a.capa[(size_t)ra * (size_t)mx + (size_t)cxa];
-      if constexpr (SPLIT) kapx = a.capa[(size_t)ry * (size_t)mx + (size_t)cxa];
-      else kapx = kap;
+      if constexpr (P::NAUX > 0) b = scalar_ptr(a.aux + (size_t)ra * (size_t)mx)[(unsigned)cxa];
+      if constexpr (CAPA) {
+        kap = (a.capa + (size_t)ra * (size_t)mx)[(unsigned)cxa];
+        if constexpr (SPLIT) kapx = (a.capa + (size_t)ry * (size_t)mx)[(unsigned)cxa];
+        else kapx = kap;
+      }
     }
   };
   auto apply_flips = [&](T q[NEQ], bool fy) {
-    if (!walls) return;
+    if (PAD || !(xflips || fy)) return;
+    asm volatile("");  // a branch, not selects on every row
+    const bool f[4] = {fx0 != (fy && a.rfy == 0), fx1 != (fy && a.rfy == 1), fx2 != (fy && a.rfy == 2),
+                       fx3 != (fy && a.rfy == 3)};
 #pragma unroll
-    for (int m = 0; m < NEQ; ++m) {
-      const bool neg = (fx && m == a.rfx) != (fy && m == a.rfy);
-      q[m] = neg ? -q[m] : q[m];
-    }
+    for (int m = 0; m < NEQ; ++m) q[m] = f[m] ? -q[m] : q[m];
   };
 
   // CFL speed of an interface: max |s| / kappa over its waves, a right-going wave against the
@@ -448,10 +533,11 @@ __device__ __forceinline__ ItemMax march_item(const StepArgs<T, P>& a, const T* 
   // FP64: plain max plus a NaN flag folded in once at the end (the same result as a
   // NaN-propagating max at every update, in two instructions instead of five)
   constexpr bool kNanFlag = sizeof(T) == 8;
-  bool nanx = false, nany = false;
-  bool bad = false;
+  unsigned long long nanx = 0, nany = 0;  // lanes that saw a NaN speed, and a bad stored cell
+  unsigned long long bad = 0;
   Cell cprev = {};
-  Iface fyprev;
+  Iface fyprev = {};
+  bool yplain = true;  // fyprev is plain (P::plain) on every lane that finishes it
   T yup[NW];  // y: alpha_p of interface R-2 times e_p(R-2).e_p(R-1), the upwind term of R-1
   T qm2[NEQ], qnext[NEQ];  // q of row R-2 (the row being finished), prefetched row R+1
   T acc0[NEQ], acc1[NEQ], acc2[NEQ], acc3[NEQ];
@@ -469,9 +555,9 @@ __device__ __forceinline__ ItemMax march_item(const StepArgs<T, P>& a, const T* 
   const int rlo = SWEEP == 1 ? y0 : y0 - 2, rhi = SWEEP == 1 ? y1 - 1 : y1 + 1;
   bool fnext;
   T bnext = T(0), knext = T(1), kxnext = T(1);
-  load_row(rlo, qnext, fnext, bnext, knext, kxnext);
-  // One marched row.  ST (steady): a row y0+2..y1-1 of the full step, for which every row test
-  // below holds, so that copy of the body is one straight block the scheduler can interleave
+  load_row(rlo, qnext, fnext, bnext, knext, kxnext, std::false_type{});
+  // One marched row.  ST (steady): a row y0+2..y1-1 of the full step whose next row is in the grid
+  // too, for which every row test below holds, so that copy of the body is one straight block the scheduler can interleave
   // (shallow water: 2.4% faster in FP64 on MI355X; the Euler kernel would spill, so it keeps one
   // copy of the body).
   auto row = [&](const int R, auto steady_tag) {
@@ -486,8 +572,8 @@ __device__ __forceinline__ ItemMax march_item(const StepArgs<T, P>& a, const T* 
       rkR = frcp(knext);
       rkX = SPLIT ? frcp(kxnext) : rkR;
     }
-    apply_flips(qR, fnext);
-    if (ST || R < rhi) load_row(R + 1, qnext, fnext, bnext, knext, kxnext);
+    apply_flips(qR, ST ? false : fnext);
+    if (ST || R < rhi) load_row(R + 1, qnext, fnext, bnext, knext, kxnext, steady_tag);
     const Cell cR = prep_cell<P>(qR, bR, a.par);
 
     // ---- request the left neighbour's cell data for the x-interfaces of row R now, so that the
@@ -506,27 +592,30 @@ __device__ __forceinline__ ItemMax march_item(const StepArgs<T, P>& a, const T* 
     T rkLx = T(1);  // 1/kappa of the left cell of the row's x-interface
     if constexpr (CAPA && SWEEP != 2) rkLx = from_left<DPP, T, DPPZ>(rkX);
 
-    // ---- y-sweep part of row R: the y-interface between rows R-1 and R (in-lane), then the
-    // y-interface one row lower, whose limiter needed it.  cY is the cell data the y-sweeps see:
+    // ---- y-interface R (between rows R-1 and R), in-lane.  cY is the cell data the y-sweeps see:
     // q^n for the unsplit step, the x-swept q* for the dimensionally split one.
     Iface fynew;
-    auto y_part = [&](const Cell& cY) {
-      // ---- y-interface R (between rows R-1 and R), in-lane
+    bool nplain = true;
+    auto y_iface = [&](const Cell& cY) {
       if (ST || R >= y0 - 1) {
         P::template rpn2<1>(cprev, cY, a.par, fynew);
         // split step: the y-speeds come from q*, which a rejected attempt (too large a dt) can
         // leave with negative depths; as in the reference's max, NaN speeds are skipped (a NaN
         // in an accepted state is still caught by the stored-cell check)
-        if ((SPLIT ? own_col : ycfl_col) && (ST || (R >= 0 && R <= my)))
-        {
+        if (ST || (R >= 0 && R <= my)) {  // (the lanes that do not count are left out at the end)
           const T sp = SPLIT ? cfl_speed_q_star(fynew, rkprev, rkR) : cfl_speed(fynew, rkprev, rkR);
           if constexpr (SPLIT) smy = vmax(smy, sp);
-          else if constexpr (kNanFlag) { smy = vmax(smy, sp); nany |= sp != sp; }
+          else if constexpr (kNanFlag) { smy = vmax(smy, sp); nany |= lanes(sp != sp); }
           else smy = nmax(smy, sp);
         }
+        nplain = (~P::template plain<1, TRANS>(cprev, cY, a.par, fynew) & kYLanes) == 0ull;
       }
+    };
 
-      // ---- finish y-interface R-1 (between rows R-2 and R-1)
+    // ---- finish y-interface R-1 (between rows R-2 and R-1), whose limiter needed interface R, and
+    // with it the cells of row R-2.  PL: the interface is plain on every lane that needs it.
+    auto y_finish = [&](auto plain_tag) {
+      constexpr bool PL = decltype(plain_tag)::value;
       if (ST || R >= y0) {
         T lp[NL], ln[NL], mR[NW];
         P::lim(fyprev, lp);
@@ -534,8 +623,16 @@ __device__ __forceinline__ ItemMax march_item(const StepArgs<T, P>& a, const T* 
         P::mdot(lp, ln, mR);
         if (ST || R >= y0 + 1) {
           T LX[NEQ], LG1[NEQ], LG2[NEQ], RX[NEQ], RG1[NEQ], RG2[NEQ];
-          finish_iface<T, P, LIM, TWC, CAPA>(fyprev, yup, fynew.al, mR, dtdy, dtdx, a, LX, LG1,
-                                             LG2, RX, RG1, RG2, rkm2, rkprev);
+          if constexpr (PL) {
+            finish_plain<T, P, LIM, TWC, CAPA>(fyprev, yup, fynew.al, mR, dtdy, dtdx, a, LX, LG1, LG2, RX, RG1,
+                                               RG2, rkm2, rkprev);
+          } else {
+            // the lower cell's data again from its state: only interfaces that are not plain need it
+            T sf[NW];
+            P::template fix<1>(prep_cell<P>(qm2, T(0), a.par), cprev, a.par, fyprev, sf);
+            finish_iface<T, P, LIM, TWC, CAPA>(fyprev, sf, yup, fynew.al, mR, dtdy, dtdx, a, LX, LG1, LG2, RX,
+                                               RG1, RG2, rkm2, rkprev);
+          }
           yswap<NEQ>(LX); yswap<NEQ>(LG1); yswap<NEQ>(LG2);
           yswap<NEQ>(RX); yswap<NEQ>(RG1); yswap<NEQ>(RG2);
           if constexpr (kImmY) {
@@ -569,13 +666,13 @@ __device__ __forceinline__ ItemMax march_item(const StepArgs<T, P>& a, const T* 
             }
             if (own_col) {
               T qn[NEQ];
-              const size_t off = (size_t)(R - 2) * (size_t)mx + (size_t)c;
+              T* const qrow = qout + (size_t)(R - 2) * (size_t)mx;
   #pragma unroll
               for (int m = 0; m < NEQ; ++m) {
                 qn[m] = CAPA ? qm2[m] + acc0[m] * rkm2 : qm2[m] + acc0[m];
-                qout[(size_t)m * plane + off] = qn[m];
+                scalar_ptr(qrow + (size_t)m * plane)[(unsigned)c] = qn[m];
               }
-              bad |= P::bad(qn, a.par);
+              bad |= lanes(P::bad(qn, a.par));
             }
           }
           if constexpr (!kImmY) {
@@ -588,45 +685,55 @@ __device__ __forceinline__ ItemMax march_item(const StepArgs<T, P>& a, const T* 
           yup[p] = P::unit_m(p) ? fyprev.al[p] : fyprev.al[p] * mR[p];
         }
       }
-
-
     };
-
-    if constexpr (!SPLIT) y_part(cR);
 
     // ---- x-interfaces of row R (the left cells were requested before the y work).  Split step:
     // every marched row (the y-sweeps need q* of the halo rows too); ghost rows are x-swept from
     // their mapped source rows, which equals refilling the ghosts of q* for extrap, periodic and
     // wall conditions.
+    const bool xrow = SWEEP != 2 && (SPLIT || ST || (R >= y0 - 1 && R <= y1));
     Cell cY = cR;
-    if (SWEEP != 2 && (SPLIT || ST || (R >= y0 - 1 && R <= y1))) {
-      const Cell cL = P::unpack(pl);
-      Iface fxi;
+    Cell cL;
+    Iface fxi;
+    bool xplain = true;
+    auto x_iface = [&]() {
+      cL = P::unpack(pl);
       P::template rpn2<0>(cL, cR, a.par, fxi);
-      if (xcfl_col && (ST || (SPLIT ? (R >= 0 && R < my) : (R >= -1 && R <= my))))
-      {
+      if (ST || (SPLIT ? (R >= 0 && R < my) : (R >= -1 && R <= my))) {
         const T sp = cfl_speed(fxi, rkLx, rkX);
-        if constexpr (kNanFlag) { smx = vmax(smx, sp); nanx |= sp != sp; }
+        if constexpr (kNanFlag) { smx = vmax(smx, sp); nanx |= lanes(sp != sp); }
         else smx = nmax(smx, sp);
       }
+      xplain = (~P::template plain<0, TRANS>(cL, cR, a.par, fxi) & kXLanes) == 0ull;
+    };
+    auto x_finish = [&](auto plain_tag) {
+      constexpr bool PL = decltype(plain_tag)::value;
       // limiter partners.  The right neighbour's wave data come over one exchange; this lane
       // forms the eigenvector products m_p of its pair (this, right) and hands the right
       // neighbour the product it needs when its wave p is right-going, alpha_p(this) * m_p, which
-      // is its left partner's upwind term (NW values instead of the left partner's NL).
+      // is its left partner's upwind term (NW values instead of the left partner's NL).  A plain
+      // interface's waves 1 and NW have one possible partner each.
       T lself[NL], lnb[NL], mR[NW], alR[NW], upL[NW];
       P::lim(fxi, lself);
 #pragma unroll
-      for (int k = 0; k < NL; ++k) lnb[k] = from_right<DPP, T, DPPZ>(lself[k]);
+      for (int k = 0; k < NL; ++k) lnb[k] = PL && P::lim_unused(k) ? T(0) : from_right<DPP, T, DPPZ>(lself[k]);
       P::mdot(lself, lnb, mR);
 #pragma unroll
       for (int p = 0; p < NW; ++p) {
         const T up = P::unit_m(p) ? lself[p] : lself[p] * mR[p];
-        upL[p] = from_left<DPP, T, DPPZ>(up);
+        upL[p] = PL && P::side(p) < 0 ? T(0) : from_left<DPP, T, DPPZ>(up);
         alR[p] = lnb[p];
       }
       T LX[NEQ], LG1[NEQ], LG2[NEQ], RX[NEQ], RG1[NEQ], RG2[NEQ];
-      finish_iface<T, P, LIM, TWC, CAPA>(fxi, upL, alR, mR, dtdx, dtdy, a, LX, LG1, LG2, RX, RG1, RG2,
-                                         rkLx, rkX);
+      if constexpr (PL) {
+        finish_plain<T, P, LIM, TWC, CAPA>(fxi, upL, alR, mR, dtdx, dtdy, a, LX, LG1, LG2, RX, RG1, RG2, rkLx,
+                                           rkX);
+      } else {
+        T sf[NW];
+        P::template fix<0>(cL, cR, a.par, fxi, sf);
+        finish_iface<T, P, LIM, TWC, CAPA>(fxi, sf, upL, alR, mR, dtdx, dtdy, a, LX, LG1, LG2, RX, RG1, RG2, rkLx,
+                                           rkX);
+      }
       if constexpr (SPLIT) {
         // q* of row R: the x-sweep only (no transverse terms); valid on the owned columns
         T qs[NEQ];
@@ -655,8 +762,28 @@ __device__ __forceinline__ ItemMax march_item(const StepArgs<T, P>& a, const T* 
           acc3[m] = G2;  // row R+1 has no other contribution yet
         }
       }
+    };
+    if constexpr (SPLIT) {
+      if (xrow) {
+        x_iface();
+        if (xplain) x_finish(std::true_type{});
+        else x_finish(std::false_type{});
+      }
+      if constexpr (SWEEP != 1) {
+        y_iface(cY);
+        if (yplain) y_finish(std::true_type{});
+        else y_finish(std::false_type{});
+      }
+    } else {
+      y_iface(cR);
+      if (yplain) y_finish(std::true_type{});
+      else y_finish(std::false_type{});
+      if (xrow) {
+        x_iface();
+        if (xplain) x_finish(std::true_type{});
+        else x_finish(std::false_type{});
+      }
     }
-    if constexpr (SPLIT && SWEEP != 1) y_part(cY);
 
     // ---- roll the column window (the x-sweep alone keeps no column state)
     if constexpr (SWEEP != 1) {
@@ -670,12 +797,17 @@ __device__ __forceinline__ ItemMax march_item(const StepArgs<T, P>& a, const T* 
       }
       cprev = cY;
       fyprev = fynew;
+      yplain = nplain;
       rkm2 = rkprev;
       rkprev = rkR;
     }
   };
-  if constexpr (SWEEP == 0 && NEQ == 3) {
+  // Steady rows run a copy of the row body of their own, except in the FP64 unsplit Euler kernels,
+  // which would spill (2048^2: 139.8 -> 153.1 us; FP64 split Euler 1024^2 45.5 -> 42.6 us, FP32
+  // 1501 x 1207 50.6 -> 48.1 us with it).
+  if constexpr (SWEEP == 0 && (NEQ == 3 || SPLIT || sizeof(T) == 4)) {
     int R = rlo;
+    const int ys = min(y1, my - 1);  // first row past the steady ones
     for (; R < y0 + 2 && R <= rhi; ++R) row(R, std::false_type{});
     // Issue priority from progress (segments of at least kPrioRows steady rows): 3 over the first
     // quarter of the steady rows, then 2, 1 and 0.  The wavefronts that share a SIMD start
@@ -685,8 +817,8 @@ __device__ __forceinline__ ItemMax march_item(const StepArgs<T, P>& a, const T* 
     // closer together.  Issue order only: no result bit changes.  (For FP32 it measured slower
     // while every wavefront still sent its own device-scope atomics at its end: finishing together
     // queued them; with one set per workgroup it is 7% faster at 4096^2, 10% at 8192^2.)
-    const bool prio = y1 - R >= kPrioRows;
-    const int pq = max((y1 - R) >> 2, 1);
+    const bool prio = ys - R >= kPrioRows;
+    const int pq = max((ys - R) >> 2, 1);
     int Rq = prio ? R + pq : INT_MAX, pl = 3;  // next row at which the priority steps down
     if (prio) __builtin_amdgcn_s_setprio(3);
     auto prio_at = [&](int r) {
@@ -698,16 +830,17 @@ __device__ __forceinline__ ItemMax march_item(const StepArgs<T, P>& a, const T* 
         else __builtin_amdgcn_s_setprio(0);
       }
     };
-    if constexpr (SPLIT && sizeof(T) == 8) {
-      // two steady rows per iteration: the rolling window's registers are renamed, not copied
-      // (FP64 split: -2% on MI355X, at 158 of its 168 VGPRs; the unsplit kernels would spill)
-      for (; R + 1 <= y1 - 1; R += 2) {
+    if constexpr (sizeof(T) == 8 && NEQ == 3 && (SPLIT || !P::FWAVE)) {
+      // two steady rows per iteration: the rolling window's registers are renamed, not copied (33
+      // of the unsplit row's 485 vector instructions: 4096^2 321 -> 308 us, 231 VGPRs).  Not for
+      // FP32 and the unsplit bathymetry kernel, which ran 1 to 5% slower with it.
+      for (; R + 1 < ys; R += 2) {
         prio_at(R);
         row(R, std::true_type{});
         row(R + 1, std::true_type{});
       }
     }
-    for (; R <= y1 - 1; ++R) {
+    for (; R < ys; ++R) {
       prio_at(R);
       row(R, std::true_type{});
     }
@@ -738,12 +871,15 @@ __device__ __forceinline__ ItemMax march_item(const StepArgs<T, P>& a, const T* 
   // Wave-uniform epilogue: no lane-divergent branch (a lane-0-only branch here lets the compiler
   // peel lanes 1-63 off into their own loop when this function runs inside the batched kernel's
   // work loop).  The caller folds the maxima into the control block.
+  // Lanes whose interfaces do not belong to the CFL set: x-interfaces 1..mx+1 (1-based), y-sweeps on
+  // columns 0..mx+1 (split: the owned columns).
+  const bool xcfl = lane >= 1 && c >= 0 && c <= mx, ycfl = SPLIT ? own_col : (c >= -1 && c <= mx);
+  T wx = wave_max(xcfl ? smx : T(0)), wy = wave_max(ycfl ? smy : T(0));
   if constexpr (kNanFlag) {
-    if (nanx) smx = T(NAN);
-    if (nany) smy = T(NAN);
+    if (nanx & lanes(xcfl)) wx = T(NAN);
+    if (nany & lanes(ycfl)) wy = T(NAN);
   }
-  const T wx = wave_max(smx), wy = wave_max(smy);
-  return ItemMax{uniform((double)wx), uniform((double)wy), __ballot(bad) != 0ull};
+  return ItemMax{uniform((double)wx), uniform((double)wy), bad != 0ull};
 }
 
 // The speed maxima and the status bits were written by atomics of the step's wavefronts; read
@@ -1213,6 +1349,7 @@ template <class T> static typename SweP<T>::Par swe_par(const claw2d_desc* d) {
   typename SweP<T>::Par p;
   p.g = T(d->grav);
   p.sqg = T(std::sqrt(d->grav));
+  p.sqgm = T(std::sqrt(d->grav) * (sizeof(T) == 8 ? 1.0 - 1e-12 : 1.0 - 1e-5));
   p.h0 = T(d->depth_ref);
   return p;
 }
@@ -1227,6 +1364,7 @@ template <class T> static typename EulerP<T>::Par euler_par(const claw2d_desc* d
   typename EulerP<T>::Par p;
   p.gamma = T(d->gamma);
   p.gamma1 = T(d->gamma - 1.0);
+  p.ggm = T(d->gamma * (d->gamma - 1.0) * (sizeof(T) == 8 ? 1.0 - 1e-12 : 1.0 - 1e-5));
   return p;
 }
 

@@ -61,12 +61,37 @@ __device__ __forceinline__ double frsq(double x) {
 }
 __device__ __forceinline__ float frsq(float x) { return __builtin_amdgcn_rsqf(x); }
 
-__device__ __forceinline__ double vmin(double a, double b) { return __builtin_fmin(a, b); }
-__device__ __forceinline__ float vmin(float a, float b) { return __builtin_fminf(a, b); }
-__device__ __forceinline__ double vmax(double a, double b) { return __builtin_fmax(a, b); }
-__device__ __forceinline__ float vmax(float a, float b) { return __builtin_fmaxf(a, b); }
+// Minimum and maximum (IEEE minNum/maxNum: a quiet NaN loses), and the same against 0.  Written as
+// the instructions themselves: from fmin/fmax the compiler first quiets each operand it cannot
+// prove free of signalling NaNs with a v_max x, x, which was 13 of the FP64 shallow-water row's
+// 524 vector instructions.  No value here is a signalling NaN: every operand is the result of
+// arithmetic or of a load that arithmetic has used.
+__device__ __forceinline__ double vmin(double a, double b) { double r; asm("v_min_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b)); return r; }
+__device__ __forceinline__ float vmin(float a, float b) { float r; asm("v_min_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b)); return r; }
+__device__ __forceinline__ double vmax(double a, double b) { double r; asm("v_max_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b)); return r; }
+__device__ __forceinline__ float vmax(float a, float b) { float r; asm("v_max_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b)); return r; }
+__device__ __forceinline__ double vmin0(double a) { double r; asm("v_min_f64 %0, %1, 0" : "=v"(r) : "v"(a)); return r; }
+__device__ __forceinline__ float vmin0(float a) { float r; asm("v_min_f32 %0, 0, %1" : "=v"(r) : "v"(a)); return r; }
+__device__ __forceinline__ double vmax0(double a) { double r; asm("v_max_f64 %0, %1, 0" : "=v"(r) : "v"(a)); return r; }
+__device__ __forceinline__ float vmax0(float a) { float r; asm("v_max_f32 %0, 0, %1" : "=v"(r) : "v"(a)); return r; }
+// min(|a|, b)
+__device__ __forceinline__ double vmin_abs(double a, double b) { double r; asm("v_min_f64 %0, |%1|, %2" : "=v"(r) : "v"(a), "v"(b)); return r; }
+__device__ __forceinline__ float vmin_abs(float a, float b) { float r; asm("v_min_f32 %0, |%1|, %2" : "=v"(r) : "v"(a), "v"(b)); return r; }
 __device__ __forceinline__ double vabs(double a) { return __builtin_fabs(a); }
 __device__ __forceinline__ float vabs(float a) { return __builtin_fabsf(a); }
+
+// the lanes of the wavefront for which c holds (one comparison writes the mask; masks are combined
+// by the scalar unit)
+__device__ __forceinline__ unsigned long long lanes(bool c) { return __builtin_amdgcn_ballot_w64(c); }
+
+// x with its sign flipped where s is negative (one or two 32-bit instructions, half the issue time
+// of the FP64 multiplication by +-1 that it replaces)
+__device__ __forceinline__ double flip_sign(double x, double s) {
+  return __longlong_as_double(__double_as_longlong(x) ^ (__double_as_longlong(s) & (long long)0x8000000000000000ull));
+}
+__device__ __forceinline__ float flip_sign(float x, float s) {
+  return __int_as_float(__float_as_int(x) ^ (__float_as_int(s) & (int)0x80000000u));
+}
 
 // phi(t/alpha)*alpha for limiter `meth` (ids of pyclaw/limiters/tvd.py: minmod 1, superbee 2,
 // van Leer 3, MC 4, beam-warming 5, 0 = unlimited).  alpha == 0 gives 0 (upstream skips a wave
@@ -74,13 +99,13 @@ __device__ __forceinline__ float vabs(float a) { return __builtin_fabsf(a); }
 // are evaluated on |alpha| and sign(alpha) t and the sign is put back: the same values, bit for bit,
 // as the two-branch form (negation and the factors 2 and 1/2 are exact), with no selects.
 template <class T> __device__ __forceinline__ T limited(T al, T t, int meth) {
-  const T sg = copysign(T(1), al), a = vabs(al), ts = sg * t;
+  const T ts = flip_sign(t, al);
   switch (meth) {
     case 1:  // minmod: max(0, min(1, theta))
-      return sg * vmax(T(0), vmin(a, ts));
+      return flip_sign(vmax0(vmin_abs(al, ts)), al);
     case 2: {  // superbee: max(0, min(1, 2 theta), min(2, theta))
-      const T lo = vmax(vmin(a, T(2) * ts), vmin(T(2) * a, ts));
-      return sg * vmax(T(0), lo);
+      const T lo = vmax(vmin_abs(al, T(2) * ts), vmin_abs(T(2) * al, ts));
+      return flip_sign(vmax0(lo), al);
     }
     case 3: {  // van Leer: (theta + |theta|)/(1 + |theta|)
       if (al == T(0)) return T(0);
@@ -88,8 +113,8 @@ template <class T> __device__ __forceinline__ T limited(T al, T t, int meth) {
       return al * ((th + ath) / (T(1) + ath));
     }
     case 4: {  // MC: max(0, min((1 + theta)/2, 2, 2 theta))
-      const T c = T(0.5) * (a + ts);
-      return sg * vmax(T(0), vmin(c, T(2) * vmin(a, ts)));
+      const T c = T(0.5) * (vabs(al) + ts);
+      return flip_sign(vmax0(vmin(c, T(2) * vmin_abs(al, ts))), al);
     }
     case 5: return al == T(0) ? T(0) : t;  // beam-warming: theta
     default: return al;
@@ -115,10 +140,16 @@ template <class T> struct SweP {
   static constexpr bool kRef = sizeof(T) == 4;  // stored depth is h - h0
   // e_p(A).e_p(B) is identically 1 for the shear wave
   __device__ __forceinline__ static constexpr bool unit_m(int p) { return p == 1; }
-  struct Par { T g, sqg, h0; };
+  struct Par { T g, sqg, h0, sqgm; };  // sqgm: sqrt(g), reduced (see plain)
   // per-cell: q as stored, sqrt(h), 1/sqrt(h), hu/sqrt(h), hv/sqrt(h)
   struct Cell { T q[3]; T s, rs, P, Q; };
-  struct Iface { T al[3]; T sf[3]; T u, v, a, ha; };
+  struct Iface { T al[3]; T u, v, a, ha; };
+  // which way wave p goes on a plain interface (below): -1 left, 1 right, 0 by the sign of its speed
+  __device__ __forceinline__ static constexpr int side(int p) { return p == 0 ? -1 : (p == 2 ? 1 : 0); }
+  // limiter data (lim, below) that a plain interface's neighbours do not need: the right-going strength
+  __device__ __forceinline__ static constexpr bool lim_unused(int k) { return k == 2; }
+  // left-going speed of a wave of side 0
+  __device__ __forceinline__ static T plain_fix(T s) { return vmin0(s); }
 
   // depth from a stored depth value
   __device__ __forceinline__ static T depth(T stored, const Par& pr) { return kRef ? stored + pr.h0 : stored; }
@@ -144,6 +175,7 @@ template <class T> struct SweP {
     return c;
   }
 
+  // Roe averages and wave strengths
   template <int DIR>
   __device__ __forceinline__ static void rpn2(const Cell& L, const Cell& R, const Par& pr, Iface& f) {
     constexpr int mu = DIR == 0 ? 1 : 2, mv = DIR == 0 ? 2 : 1;
@@ -158,10 +190,18 @@ template <class T> struct SweP {
     const T ha = T(0.5) * ra;
     const T d0 = R.q[0] - L.q[0], dn = R.q[mu] - L.q[mu], dt = R.q[mv] - L.q[mv];
     const T s1 = u - a, s3 = u + a;
-    const T a1 = (s3 * d0 - dn) * ha;
-    const T a2 = dt - v * d0;
-    const T a3 = (dn - s1 * d0) * ha;
-    T sf1 = vmin(s1, T(0)), sf2 = T(0), sf3 = T(0);
+    f.al[0] = (s3 * d0 - dn) * ha;
+    f.al[1] = dt - v * d0;
+    f.al[2] = (dn - s1 * d0) * ha;
+    f.u = u; f.v = v; f.a = a; f.ha = ha;
+  }
+  // left-going speed of each wave, with the entropy fix
+  template <int DIR>
+  __device__ __forceinline__ static void fix(const Cell& L, const Cell& R, const Par& pr, const Iface& f, T sf[3]) {
+    constexpr int mu = DIR == 0 ? 1 : 2;
+    const T pnL = DIR == 0 ? L.P : L.Q, pnR = DIR == 0 ? R.P : R.Q;
+    const T u = f.u, a1 = f.al[0], a3 = f.al[2], s1 = f.u - f.a, s3 = f.u + f.a;
+    T sf1 = vmin0(s1), sf2 = T(0), sf3 = T(0);
     const T s0 = pnL * L.rs - pr.sqg * L.s;  // u - c in the left cell
     if (s0 < T(0)) {
       const T h1 = depth(L.q[0] + a1, pr), hu1 = L.q[mu] + a1 * s1;
@@ -172,7 +212,7 @@ template <class T> struct SweP {
     }
     if (u < T(0)) {
       sf2 = u;
-      sf3 = vmin(s3, T(0));
+      sf3 = vmin0(s3);
       const T h3 = depth(R.q[0] - a3, pr), hu3 = R.q[mu] - a3 * s3;
       if (h3 > T(0) && hu3 < T(0) && hu3 * hu3 > pr.g * (h3 * h3) * h3) {
         const T s3r = pnR * R.rs + pr.sqg * R.s;  // u + c in the right cell
@@ -182,9 +222,27 @@ template <class T> struct SweP {
         }
       }
     }
-    f.al[0] = a1; f.al[1] = a2; f.al[2] = a3;
-    f.sf[0] = sf1; f.sf[1] = sf2; f.sf[2] = sf3;
-    f.u = u; f.v = v; f.a = a; f.ha = ha;
+    sf[0] = sf1; sf[1] = sf2; sf[2] = sf3;
+  }
+  // The lanes whose interface is plain: subsonic along the normal (|u| < a) and, where it is split transversely,
+  // across it (|v| < a), and no entropy fix applies for certain, so that fix() gives s1, min(u, 0)
+  // and 0.  The 1-wave needs the fix only if s0 = uL - cL < 0 and the middle state h1 = hL + a1,
+  // (hu)1 = (hu)L + a1 s1 has u1 > c1.  With d = a1/hL and s1 < 0,
+  //   u1 < c1  <=>  uL + d s1 < cL (1 + d)^(3/2),  and (1 + d)^(3/2) >= 1 + (3/2) d,
+  // so  a1 (1.5 cL - s1) > s0 hL  rules it out (for a1 >= 0 it always holds).  1.6 and a sound speed
+  // reduced by 1e-12 (FP32 1e-5), far more than the rounding of either side, keep the test on the
+  // safe side of fix()'s own, and where s0 >= 0 fix() takes min(s1, 0) as well.  The 3-wave's
+  // test is its mirror image.  A NaN fails every test.
+  template <int DIR, bool TRANS>
+  __device__ __forceinline__ static unsigned long long plain(const Cell& L, const Cell& R, const Par& pr,
+                                                             const Iface& f) {
+    const T pnL = DIR == 0 ? L.P : L.Q, pnR = DIR == 0 ? R.P : R.Q;
+    const T cL = pr.sqgm * L.s, cR = pr.sqgm * R.s;
+    const T pL = pnL * L.rs - cL, pR = pnR * R.rs + cR;
+    const T s1 = f.u - f.a, s3 = f.u + f.a;
+    const T w1 = f.al[0] * fma(T(1.6), cL, -s1), w3 = f.al[2] * fma(T(1.6), cR, s3);
+    return lanes(vabs(f.u) < f.a) & (TRANS ? lanes(vabs(f.v) < f.a) : ~0ull) &
+           lanes(w1 > pL * depth(L.q[0], pr)) & lanes(w3 < pR * depth(R.q[0], pr));
   }
 
   __device__ __forceinline__ static T smax(const Iface& f) { return vabs(f.u) + f.a; }
@@ -243,7 +301,7 @@ template <class T> struct SweP {
   __device__ __forceinline__ static void expand_t_split(const Iface& f, const TConst& tc, T w, const T b[NW],
                                                         T Gm[NEQ], T Gp[NEQ]) {
     const T c0 = (w * tc.vm) * b[0];
-    const T c1m = (w * vmin(f.v, T(0))) * b[1], c1p = (w * vmax(f.v, T(0))) * b[1];
+    const T c1m = (w * vmin0(f.v)) * b[1], c1p = (w * vmax0(f.v)) * b[1];
     const T c2 = (w * tc.vp) * b[2];
     Gm[0] = c0;
     Gm[1] = fma(c0, f.u, c1m);
@@ -264,11 +322,14 @@ template <class T> struct EulerP {
   static constexpr int NAUX = 0;
   static constexpr bool FWAVE = false;
   __device__ __forceinline__ static constexpr bool unit_m(int) { return false; }
-  struct Par { T gamma, gamma1; };
+  struct Par { T gamma, gamma1, ggm; };  // ggm: gamma gamma1, reduced (see plain)
   // per-cell: q, 1/sqrt(rho), rho u/sqrt(rho), rho v/sqrt(rho), (E+p)/sqrt(rho), c
   // (sqrt(rho) = rho/sqrt(rho) is formed where it is used: one register pair less per cell)
   struct Cell { T q[4]; T rs, P, Q, Hs, c; };
-  struct Iface { T al[4]; T sf[4]; T u, v, a, H, i2a; };
+  struct Iface { T al[4]; T u, v, a, H, i2a; };
+  __device__ __forceinline__ static constexpr int side(int p) { return p == 0 ? -1 : (p == 3 ? 1 : 0); }
+  __device__ __forceinline__ static constexpr bool lim_unused(int k) { return k == 3; }
+  __device__ __forceinline__ static T plain_fix(T s) { return vmin0(s); }
 
   __device__ __forceinline__ static bool bad(const T q[4], const Par&) { return !(q[0] > T(0)); }
 
@@ -335,33 +396,60 @@ template <class T> struct EulerP {
     const T as = dt - v * d0;
     const T a4 = (dn + (a - u) * d0 - a * ae) * i2a;
     const T a1 = d0 - ae - a4;
-    const T s1 = u - a, s4 = u + a;
-    T sf1 = vmin(s1, T(0)), sfu = T(0), sf4 = T(0);
+    f.al[0] = a1; f.al[1] = ae; f.al[2] = as; f.al[3] = a4;
+    f.u = u; f.v = v; f.a = a; f.H = H; f.i2a = i2a;
+  }
+  // the states right of wave 1 and left of wave 4, interface frame
+  struct Mid { T r, n, t, E; };
+  template <int DIR> __device__ __forceinline__ static Mid mid1(const Cell& L, const Iface& f) {
+    constexpr int mu = DIR == 0 ? 1 : 2, mv = DIR == 0 ? 2 : 1;
+    const T a1 = f.al[0], s1 = f.u - f.a;
+    return Mid{L.q[0] + a1, L.q[mu] + a1 * s1, L.q[mv] + a1 * f.v, L.q[3] + a1 * (f.H - f.u * f.a)};
+  }
+  template <int DIR> __device__ __forceinline__ static Mid mid4(const Cell& R, const Iface& f) {
+    constexpr int mu = DIR == 0 ? 1 : 2, mv = DIR == 0 ? 2 : 1;
+    const T a4 = f.al[3], s4 = f.u + f.a;
+    return Mid{R.q[0] - a4, R.q[mu] - a4 * s4, R.q[mv] - a4 * f.v, R.q[3] - a4 * (f.H + f.u * f.a)};
+  }
+  template <int DIR>
+  __device__ __forceinline__ static void fix(const Cell& L, const Cell& R, const Par& pr, const Iface& f, T sf[4]) {
+    const T pnL = DIR == 0 ? L.P : L.Q, pnR = DIR == 0 ? R.P : R.Q;
+    const T s1 = f.u - f.a, s4 = f.u + f.a;
+    T sf1 = vmin0(s1), sfu = T(0), sf4 = T(0);
     const T s0 = pnL * L.rs - L.c;
     if (s0 < T(0)) {
-      const T r1 = L.q[0] + a1, n1 = L.q[mu] + a1 * s1, t1 = L.q[mv] + a1 * v,
-              E1 = L.q[3] + a1 * (H - u * a);
-      if (sonic_cross(r1, n1, t1, E1, pr, true)) {
-        const T s1r = sonic_speed(r1, n1, t1, E1, pr, T(-1));
+      const Mid m = mid1<DIR>(L, f);
+      if (sonic_cross(m.r, m.n, m.t, m.E, pr, true)) {
+        const T s1r = sonic_speed(m.r, m.n, m.t, m.E, pr, T(-1));
         sf1 = s0 * (s1r - s1) / (s1r - s0);
       }
     }
-    if (u < T(0)) {
-      sfu = u;
-      sf4 = vmin(s4, T(0));
-      const T r4 = R.q[0] - a4, n4 = R.q[mu] - a4 * s4, t4 = R.q[mv] - a4 * v,
-              E4 = R.q[3] - a4 * (H + u * a);
-      if (sonic_cross(r4, n4, t4, E4, pr, false)) {
+    if (f.u < T(0)) {
+      sfu = f.u;
+      sf4 = vmin0(s4);
+      const Mid m = mid4<DIR>(R, f);
+      if (sonic_cross(m.r, m.n, m.t, m.E, pr, false)) {
         const T s4r = pnR * R.rs + R.c;
         if (s4r > T(0)) {
-          const T s4l = sonic_speed(r4, n4, t4, E4, pr, T(1));
+          const T s4l = sonic_speed(m.r, m.n, m.t, m.E, pr, T(1));
           sf4 = s4l * (s4r - s4) / (s4r - s4l);
         }
       }
     }
-    f.al[0] = a1; f.al[1] = ae; f.al[2] = as; f.al[3] = a4;
-    f.sf[0] = sf1; f.sf[1] = sfu; f.sf[2] = sfu; f.sf[3] = sf4;
-    f.u = u; f.v = v; f.a = a; f.H = H; f.i2a = i2a;
+    sf[0] = sf1; sf[1] = sfu; sf[2] = sfu; sf[3] = sf4;
+  }
+  // A plain interface (see SweP::plain): subsonic in both directions, and neither middle state
+  // can pass sonic_cross: rho > 0 and n |n| (wave 4: -n |n|) below gamma p rho, reduced by far more
+  // than the rounding of either side.
+  template <int DIR, bool TRANS>
+  __device__ __forceinline__ static unsigned long long plain(const Cell& L, const Cell& R, const Par& pr,
+                                                             const Iface& f) {
+    const Mid m1 = mid1<DIR>(L, f), m4 = mid4<DIR>(R, f);
+    const T P1 = m1.E * m1.r - T(0.5) * (m1.n * m1.n + m1.t * m1.t);
+    const T P4 = m4.E * m4.r - T(0.5) * (m4.n * m4.n + m4.t * m4.t);
+    return lanes(vabs(f.u) < f.a) & (TRANS ? lanes(vabs(f.v) < f.a) : ~0ull) & lanes(m1.r > T(0)) &
+           lanes(m4.r > T(0)) & lanes(m1.n * vabs(m1.n) < pr.ggm * P1) &
+           lanes(-m4.n * vabs(m4.n) < pr.ggm * P4);
   }
 
   __device__ __forceinline__ static T smax(const Iface& f) { return vabs(f.u) + f.a; }
@@ -448,7 +536,7 @@ template <class T> struct EulerP {
                                                         T Gm[NEQ], T Gp[NEQ]) {
     {
 #pragma clang fp contract(off)
-      const T wvm = w * vmin(f.v, T(0)), wvp = w * vmax(f.v, T(0));
+      const T wvm = w * vmin0(f.v), wvp = w * vmax0(f.v);
       const T c0 = (w * tc.vm) * b[0], c3 = (w * tc.vp) * b[3];
       const T c1m = wvm * b[1], c2m = wvm * b[2], c1p = wvp * b[1], c2p = wvp * b[2];
       Gm[0] = c0 + c1m;
@@ -512,6 +600,19 @@ template <class T> struct SweBathyP : SweP<T> {
     return s < T(0) ? T(1) : (s > T(0) ? T(0) : T(0.5));
   }
 
+  __device__ __forceinline__ static T plain_fix(T s) { return left_frac(s); }
+  template <int DIR>
+  __device__ __forceinline__ static void fix(const Cell&, const Cell&, const Par&, const Iface& f, T sf[3]) {
+    sf[0] = left_frac(f.u - f.a);
+    sf[1] = left_frac(f.u);
+    sf[2] = left_frac(f.u + f.a);
+  }
+  // no entropy fix: a plain interface is subsonic in both directions (so at least one cell is wet)
+  template <int DIR, bool TRANS>
+  __device__ __forceinline__ static unsigned long long plain(const Cell&, const Cell&, const Par&, const Iface& f) {
+    return lanes(vabs(f.u) < f.a) & (TRANS ? lanes(vabs(f.v) < f.a) : ~0ull);
+  }
+
   template <int DIR>
   __device__ __forceinline__ static void rpn2(const Cell& L, const Cell& R, const Par& pr, Iface& f) {
     const T pnL = DIR == 0 ? L.P : L.Q, ptL = DIR == 0 ? L.Q : L.P;
@@ -540,9 +641,6 @@ template <class T> struct SweBathyP : SweP<T> {
     f.al[0] = (s3 * d1 - d2) * ha;
     f.al[1] = d3 - v * d1;
     f.al[2] = (d2 - s1 * d1) * ha;
-    f.sf[0] = left_frac(s1);
-    f.sf[1] = left_frac(u);
-    f.sf[2] = left_frac(s3);
     f.u = u; f.v = v; f.a = a; f.ha = ha;
   }
 };
