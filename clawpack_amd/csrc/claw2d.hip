@@ -537,6 +537,13 @@ __device__ __forceinline__ ItemMax march_item(const StepArgs<T, P>& a, const T* 
   unsigned long long bad = 0;
   Cell cprev = {};
   Iface fyprev = {};
+  // Euler's test for plain interfaces is the longest (two middle states), and where the flow is
+  // transonic or supersonic it fails row after row: a direction whose row was not plain is taken
+  // as not plain for the next rows too and tested again kRetry rows later (2048^2 FP64 with
+  // Mach 2.5 flow: 162 -> 150 us, subsonic unchanged; the split step's and shallow water's shorter
+  // tests are made every row)
+  constexpr int kRetry = NEQ == 4 && !SPLIT ? 4 : 0;
+  int yretry = INT_MIN, xretry = INT_MIN;
   bool yplain = true;  // fyprev is plain (P::plain) on every lane that finishes it
   T yup[NW];  // y: alpha_p of interface R-2 times e_p(R-2).e_p(R-1), the upwind term of R-1
   T qm2[NEQ], qnext[NEQ];  // q of row R-2 (the row being finished), prefetched row R+1
@@ -608,7 +615,12 @@ __device__ __forceinline__ ItemMax march_item(const StepArgs<T, P>& a, const T* 
           else if constexpr (kNanFlag) { smy = vmax(smy, sp); nany |= lanes(sp != sp); }
           else smy = nmax(smy, sp);
         }
-        nplain = (~P::template plain<1, TRANS>(cprev, cY, a.par, fynew) & kYLanes) == 0ull;
+        if (kRetry > 0 && R < yretry) {
+          nplain = false;
+        } else {
+          nplain = P::template plain<1, TRANS>(cprev, cY, a.par, fynew, kYLanes);
+          if (kRetry > 0 && !nplain) yretry = R + kRetry;
+        }
       }
     };
 
@@ -704,7 +716,12 @@ __device__ __forceinline__ ItemMax march_item(const StepArgs<T, P>& a, const T* 
         if constexpr (kNanFlag) { smx = vmax(smx, sp); nanx |= lanes(sp != sp); }
         else smx = nmax(smx, sp);
       }
-      xplain = (~P::template plain<0, TRANS>(cL, cR, a.par, fxi) & kXLanes) == 0ull;
+      if (kRetry > 0 && R < xretry) {
+        xplain = false;
+      } else {
+        xplain = P::template plain<0, TRANS>(cL, cR, a.par, fxi, kXLanes);
+        if (kRetry > 0 && !xplain) xretry = R + kRetry;
+      }
     };
     auto x_finish = [&](auto plain_tag) {
       constexpr bool PL = decltype(plain_tag)::value;
@@ -802,10 +819,10 @@ __device__ __forceinline__ ItemMax march_item(const StepArgs<T, P>& a, const T* 
       rkprev = rkR;
     }
   };
-  // Steady rows run a copy of the row body of their own, except in the FP64 unsplit Euler kernels,
-  // which would spill (2048^2: 139.8 -> 153.1 us; FP64 split Euler 1024^2 45.5 -> 42.6 us, FP32
-  // 1501 x 1207 50.6 -> 48.1 us with it).
-  if constexpr (SWEEP == 0 && (NEQ == 3 || SPLIT || sizeof(T) == 4)) {
+  // Steady rows run a copy of the row body of their own, except in the unsplit Euler kernels: FP64
+  // would spill (2048^2: 139.8 -> 153.1 us), and FP32 gains where the flow is subsonic (1501 x 1207
+  // 51.2 -> 48.9 us) but loses where it is not (2048^2 88.0 -> 94.1 us).
+  if constexpr (SWEEP == 0 && (NEQ == 3 || SPLIT)) {
     int R = rlo;
     const int ys = min(y1, my - 1);  // first row past the steady ones
     for (; R < y0 + 2 && R <= rhi; ++R) row(R, std::false_type{});
@@ -1167,16 +1184,19 @@ __global__ void __launch_bounds__(64) mass_final(const double* part, double* out
 
 // ------------------------------------------------------------------------------------------
 // Step kernels instantiated in translation units of their own (claw2d_swe32.hip,
-// claw2d_euler64.hip, claw2d_euler32.hip), which are built with another LLVM machine scheduler
-// (clawpack_amd/build.py: FP32 shallow water -2.7% and FP32 Euler -1.1% with max-ilp, FP64 Euler
-// -2.6% and no spill with iterative-minreg on MI355X; the same schedulers made other kernels up to
-// 6% slower).  The host code below launches them through their kernel handles, which those units
-// register with their own device code.  Scheduling does not change the arithmetic: contraction is
-// decided per source expression.
+// claw2d_euler64.hip, claw2d_euler32.hip), which are built with LLVM's max-ilp machine scheduler
+// (clawpack_amd/build.py has the figures; it made other kernels up to 6% slower).  The host code
+// below launches them through their kernel handles, which those units register with their own
+// device code.  Scheduling does not change the arithmetic: contraction is decided per source
+// expression.
 extern template __global__ void step2_fused<float, SweP<float>, 4, false, 2, false, 0, false>(
     StepArgs<float, SweP<float>>);
-extern template __global__ void step2_fused<double, EulerP<double>, 4, false, 2, false, 0, false>(
-    StepArgs<double, EulerP<double>>);
+#define CLAW_EULER64_KERNELS(K)                                          \
+  K(4, 2) K(4, 1) K(1, 2) K(1, 1) K(0, -1)
+#define CLAW_EULER64_EXTERN(LIM, TWC)                                                               \
+  extern template __global__ void step2_fused<double, EulerP<double>, LIM, false, TWC, false, 0, false>( \
+      StepArgs<double, EulerP<double>>);
+CLAW_EULER64_KERNELS(CLAW_EULER64_EXTERN)
 extern template __global__ void step2_fused<float, EulerP<float>, 4, false, 2, false, 0, false>(
     StepArgs<float, EulerP<float>>);
 

@@ -1,11 +1,12 @@
-// The FP64 Euler step kernel for the MC limiter at order 2 with transverse_waves = 2 (the bench's
-// Euler kernel), in a translation unit of its own so that it can be built with LLVM's
-// iterative-minreg machine scheduler, which fits it in 256 VGPRs without the spill the default
-// scheduler leaves (clawpack_amd/build.py).  claw2d.hip declares it extern and launches it.
+// The FP64 unsplit Euler step kernels (plain and periodic boundaries, no capacity function), in a
+// translation unit of their own so that they can be built with LLVM's max-ilp machine scheduler
+// (clawpack_amd/build.py).  claw2d.hip declares them extern and launches them.
 #define CLAW_KERNEL_UNIT 1
 #include "claw2d.hip"
 
 namespace claw {
-template __global__ void step2_fused<double, EulerP<double>, 4, false, 2, false, 0, false>(
-    StepArgs<double, EulerP<double>>);
+#define CLAW_EULER64_DEFINE(LIM, TWC)                                                        \
+  template __global__ void step2_fused<double, EulerP<double>, LIM, false, TWC, false, 0, false>( \
+      StepArgs<double, EulerP<double>>);
+CLAW_EULER64_KERNELS(CLAW_EULER64_DEFINE)
 }  // namespace claw

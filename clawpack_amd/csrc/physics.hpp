@@ -84,6 +84,9 @@ __device__ __forceinline__ float vabs(float a) { return __builtin_fabsf(a); }
 // by the scalar unit)
 __device__ __forceinline__ unsigned long long lanes(bool c) { return __builtin_amdgcn_ballot_w64(c); }
 
+// every lane of `need` is in `mask`
+__device__ __forceinline__ bool covers(unsigned long long mask, unsigned long long need) { return (~mask & need) == 0ull; }
+
 // x with its sign flipped where s is negative (one or two 32-bit instructions, half the issue time
 // of the FP64 multiplication by +-1 that it replaces)
 __device__ __forceinline__ double flip_sign(double x, double s) {
@@ -224,7 +227,11 @@ template <class T> struct SweP {
     }
     sf[0] = sf1; sf[1] = sf2; sf[2] = sf3;
   }
-  // The lanes whose interface is plain: subsonic along the normal (|u| < a) and, where it is split transversely,
+  // the lanes with |u| < a and, where the interface is split transversely, |v| < a
+  template <bool TRANS> __device__ __forceinline__ static unsigned long long subsonic(const Iface& f) {
+    return lanes(vabs(f.u) < f.a) & (TRANS ? lanes(vabs(f.v) < f.a) : ~0ull);
+  }
+  // Whether the interfaces of the lanes `need` are all plain: subsonic along the normal (|u| < a) and, where it is split transversely,
   // across it (|v| < a), and no entropy fix applies for certain, so that fix() gives s1, min(u, 0)
   // and 0.  The 1-wave needs the fix only if s0 = uL - cL < 0 and the middle state h1 = hL + a1,
   // (hu)1 = (hu)L + a1 s1 has u1 > c1.  With d = a1/hL and s1 < 0,
@@ -234,15 +241,15 @@ template <class T> struct SweP {
   // safe side of fix()'s own, and where s0 >= 0 fix() takes min(s1, 0) as well.  The 3-wave's
   // test is its mirror image.  A NaN fails every test.
   template <int DIR, bool TRANS>
-  __device__ __forceinline__ static unsigned long long plain(const Cell& L, const Cell& R, const Par& pr,
-                                                             const Iface& f) {
+  __device__ __forceinline__ static bool plain(const Cell& L, const Cell& R, const Par& pr, const Iface& f,
+                                               unsigned long long need) {
     const T pnL = DIR == 0 ? L.P : L.Q, pnR = DIR == 0 ? R.P : R.Q;
     const T cL = pr.sqgm * L.s, cR = pr.sqgm * R.s;
     const T pL = pnL * L.rs - cL, pR = pnR * R.rs + cR;
     const T s1 = f.u - f.a, s3 = f.u + f.a;
     const T w1 = f.al[0] * fma(T(1.6), cL, -s1), w3 = f.al[2] * fma(T(1.6), cR, s3);
-    return lanes(vabs(f.u) < f.a) & (TRANS ? lanes(vabs(f.v) < f.a) : ~0ull) &
-           lanes(w1 > pL * depth(L.q[0], pr)) & lanes(w3 < pR * depth(R.q[0], pr));
+    return covers(subsonic<TRANS>(f) & lanes(w1 > pL * depth(L.q[0], pr)) & lanes(w3 < pR * depth(R.q[0], pr)),
+                  need);
   }
 
   __device__ __forceinline__ static T smax(const Iface& f) { return vabs(f.u) + f.a; }
@@ -438,18 +445,23 @@ template <class T> struct EulerP {
     }
     sf[0] = sf1; sf[1] = sfu; sf[2] = sfu; sf[3] = sf4;
   }
+  // the lanes with |u| < a and, where the interface is split transversely, |v| < a
+  template <bool TRANS> __device__ __forceinline__ static unsigned long long subsonic(const Iface& f) {
+    return lanes(vabs(f.u) < f.a) & (TRANS ? lanes(vabs(f.v) < f.a) : ~0ull);
+  }
   // A plain interface (see SweP::plain): subsonic in both directions, and neither middle state
   // can pass sonic_cross: rho > 0 and n |n| (wave 4: -n |n|) below gamma p rho, reduced by far more
   // than the rounding of either side.
   template <int DIR, bool TRANS>
-  __device__ __forceinline__ static unsigned long long plain(const Cell& L, const Cell& R, const Par& pr,
-                                                             const Iface& f) {
+  __device__ __forceinline__ static bool plain(const Cell& L, const Cell& R, const Par& pr, const Iface& f,
+                                               unsigned long long need) {
+    // (unsplit: the middle states are left out where the flow is not subsonic)
+    if (TRANS && !covers(subsonic<TRANS>(f), need)) return false;
     const Mid m1 = mid1<DIR>(L, f), m4 = mid4<DIR>(R, f);
     const T P1 = m1.E * m1.r - T(0.5) * (m1.n * m1.n + m1.t * m1.t);
     const T P4 = m4.E * m4.r - T(0.5) * (m4.n * m4.n + m4.t * m4.t);
-    return lanes(vabs(f.u) < f.a) & (TRANS ? lanes(vabs(f.v) < f.a) : ~0ull) & lanes(m1.r > T(0)) &
-           lanes(m4.r > T(0)) & lanes(m1.n * vabs(m1.n) < pr.ggm * P1) &
-           lanes(-m4.n * vabs(m4.n) < pr.ggm * P4);
+    return covers((TRANS ? ~0ull : subsonic<TRANS>(f)) & lanes(m1.r > T(0)) & lanes(m4.r > T(0)) & lanes(m1.n * vabs(m1.n) < pr.ggm * P1) &
+                      lanes(-m4.n * vabs(m4.n) < pr.ggm * P4), need);
   }
 
   __device__ __forceinline__ static T smax(const Iface& f) { return vabs(f.u) + f.a; }
@@ -609,8 +621,9 @@ template <class T> struct SweBathyP : SweP<T> {
   }
   // no entropy fix: a plain interface is subsonic in both directions (so at least one cell is wet)
   template <int DIR, bool TRANS>
-  __device__ __forceinline__ static unsigned long long plain(const Cell&, const Cell&, const Par&, const Iface& f) {
-    return lanes(vabs(f.u) < f.a) & (TRANS ? lanes(vabs(f.v) < f.a) : ~0ull);
+  __device__ __forceinline__ static bool plain(const Cell&, const Cell&, const Par&, const Iface& f,
+                                               unsigned long long need) {
+    return covers(SweP<T>::template subsonic<TRANS>(f), need);
   }
 
   template <int DIR>
