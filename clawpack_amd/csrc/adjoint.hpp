@@ -27,19 +27,31 @@
 namespace claw {
 namespace adj {
 
-// Reciprocal: IEEE on the host, hardware estimate + two Newton steps on the device (the adjoint
-// only needs accuracy far below its 1e-6 gradient tolerance).
+// Reciprocal and reciprocal square root: IEEE on the host, the hardware estimate and one third-order
+// step on the device (as frcp and frsq of physics.hpp: about 1 ulp).
 __host__ __device__ inline double arcp(double x) {
 #if defined(__HIP_DEVICE_COMPILE__)
-  double r = __builtin_amdgcn_rcp(x);
-  r = fma(fma(-x, r, 1.0), r, r);
-  r = fma(fma(-x, r, 1.0), r, r);
-  return r;
+  const double r = __builtin_amdgcn_rcp(x), e = fma(-x, r, 1.0);
+  return fma(r, fma(e, e, e), r);
 #else
   return 1.0 / x;
 #endif
 }
+__host__ __device__ inline double arsq(double x) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  const double r = __builtin_amdgcn_rsq(x), e = fma(-(x * r), r, 1.0);
+  return fma(r * e, fma(0.375, e, 0.5), r);
+#else
+  return 1.0 / sqrt(x);
+#endif
+}
 __host__ __device__ inline double asqrt(double x) { return sqrt(x); }
+#if defined(__HIPCC__)
+// x with its sign flipped where s is negative
+__device__ inline double flip_sign(double x, double s) {
+  return __longlong_as_double(__double_as_longlong(x) ^ (__double_as_longlong(s) & (long long)0x8000000000000000ull));
+}
+#endif
 
 struct CellF {
   double h, hn, ht, s, r, P, Q;  // s = sqrt(h), r = 1/s, P = hn*r, Q = ht*r
@@ -51,8 +63,8 @@ struct CellB {
 __host__ __device__ inline CellF cell_fwd(double h, double hn, double ht) {
   CellF c;
   c.h = h; c.hn = hn; c.ht = ht;
-  c.s = asqrt(h);
-  c.r = arcp(c.s);
+  c.r = arsq(h);
+  c.s = h * c.r;
   c.P = hn * c.r;
   c.Q = ht * c.r;
   return c;
@@ -84,8 +96,9 @@ __host__ __device__ inline WaveF wave_fwd(const CellF& L, const CellF& R, double
   w.inv = arcp(w.S);
   w.u = (L.P + R.P) * w.inv;
   w.v = (L.Q + R.Q) * w.inv;
-  w.a = asqrt(g * ((L.h + R.h) * 0.5));
-  w.ha = 0.5 * arcp(w.a);
+  const double gh = g * ((L.h + R.h) * 0.5), ra = arsq(gh);
+  w.a = gh * ra;
+  w.ha = 0.5 * ra;
   w.d0 = R.h - L.h;
   w.dn = R.hn - L.hn;
   w.dt = R.ht - L.ht;
@@ -119,7 +132,7 @@ __host__ __device__ inline void wave_rev(const CellF& L, const CellF& R, const W
   b.u += b.s1 + b.s3;
   b.a += b.s3 - b.s1;
   // ha = 0.5/a, a = sqrt(g*(hL + hR)/2): d a / d(gh) = 0.5/a = ha
-  b.a -= b.ha * w.ha * arcp(w.a);
+  b.a -= b.ha * (2.0 * w.ha * w.ha);  // 1/a = 2 ha
   const double ghb = b.a * w.ha;
   Lb.h += ghb * 0.5 * g;
   Rb.h += ghb * 0.5 * g;
@@ -493,6 +506,146 @@ __host__ __device__ inline void iface_core(const CellF& L, const CellF& R, const
   Wb.a2 += alb[1];
   Wb.a3 += alb[2];
 }
+
+#if defined(__HIPCC__)
+// The lanes whose interface is plain (as SweP::plain of physics.hpp: subsonic along and across, and
+// no entropy fix applies for certain; sqgm is sqrt(g) reduced as there).  fix_fwd then gives the
+// fractions s1, min(u, 0) and 0.
+__device__ inline unsigned long long plain_lanes(const CellF& L, const CellF& R, const WaveF& w, double sqgm) {
+  const double cL = sqgm * L.s, cR = sqgm * R.s;
+  const double pL = L.P * L.r - cL, pR = R.P * R.r + cR;
+  const double w1 = w.a1 * fma(1.6, cL, -w.s1), w3 = w.a3 * fma(1.6, cR, w.s3);
+  return __builtin_amdgcn_ballot_w64(fabs(w.u) < w.a) & __builtin_amdgcn_ballot_w64(fabs(w.v) < w.a) &
+         __builtin_amdgcn_ballot_w64(w1 > pL * L.h) & __builtin_amdgcn_ballot_w64(w3 < pR * R.h);
+}
+
+// limited_d for minmod and MC without branches: evaluated on |al| and sign(al) t (both are odd in
+// (al, t)), the same partials on the same branch.
+template <int LIM> __device__ inline double limited_dn(double al, double t, double& dal, double& dt) {
+  static_assert(LIM == 1 || LIM == 4, "minmod or MC");
+  const double A = fabs(al), U = flip_sign(t, al);
+  double v, da, du;
+  if (LIM == 1) {
+    const bool x = A < U;
+    v = x ? A : U;
+    da = x ? 1.0 : 0.0;
+    du = x ? 0.0 : 1.0;
+  } else {
+    v = 0.5 * (A + U);
+    const double t2 = 2.0 * U, a2 = 2.0 * A;
+    const bool kt = t2 < v;
+    v = kt ? t2 : v;
+    const bool ka = a2 < v;
+    v = ka ? a2 : v;
+    da = ka ? 2.0 : (kt ? 0.0 : 0.5);
+    du = ka ? 0.0 : (kt ? 2.0 : 0.5);
+  }
+  const bool on = v > 0.0;
+  dal = on ? da : 0.0;
+  dt = on ? du : 0.0;
+  return on ? flip_sign(v, al) : 0.0;
+}
+
+// iface_core for a plain interface at order 2 with transverse_waves 2: wave 1 goes left (its limiter
+// partner is the right interface), wave 3 right, the shear wave by the sign of u; the transverse
+// speeds v - a and v + a have fixed signs.  NLb and NRb get only what such waves read: a2, a3, s3, v
+// of the left interface and a1, a2, s1, v of the right one.
+template <int LIM>
+__device__ inline void iface_plain(const WaveF& w, const LimD& nl, const LimD& nr, const double bLX[3],
+                                   const double bLG1[3], const double bLG2[3], const double bRX[3],
+                                   const double bRG1[3], const double bRG2[3], double r, double rt, WaveB& Wb,
+                                   LimD& NLb, LimD& NRb) {
+  // ---- forward values
+  const double vv1 = 1.0 + w.v * w.v, n1 = w.s1 * w.s1 + vv1, n3 = w.s3 * w.s3 + vv1;
+  const double rn = arcp(n1 * n3), in0 = n3 * rn, in2 = n1 * rn;
+  const double mr0 = 1.0 + w.s1 * nr.s1 + w.v * nr.v, ml2 = 1.0 + nl.s3 * w.s3 + nl.v * w.v;
+  const bool right = w.u > 0.0, uneg = w.u < 0.0;
+  const double U0 = nr.a1 * mr0, U1 = right ? nl.a2 : nr.a2, U2 = nl.a3 * ml2;
+  double da0, dt0, da1, dt1, da2, dt2;
+  const double p0 = limited_dn<LIM>(w.a1, U0 * in0, da0, dt0);
+  const double p1 = limited_dn<LIM>(w.a2, U1, da1, dt1);
+  const double p2 = limited_dn<LIM>(w.a3, U2 * in2, da2, dt2);
+  const double au = fabs(w.u);
+  const double c0 = -w.s1 * (1.0 + w.s1 * r), c1 = au * (1.0 - au * r), c2 = w.s3 * (1.0 - w.s3 * r);
+  const double k0 = c0 * p0, k1 = c1 * p1, k2 = c2 * p2;
+  const double ul = uneg ? w.u : 0.0, ur = uneg ? 0.0 : w.u;
+  const double e0 = w.s1 * w.a1, q2 = w.s3 * w.a3;
+  const double A0 = e0 + k0, A1 = ul * w.a2 + k1, A2 = k2;
+  const double B0 = -k0, B1 = ur * w.a2 - k1, B2 = q2 - k2;
+  // ---- LX, RX
+  const double XL0 = -r * (e0 + 0.5 * k0), XL2 = -(0.5 * r) * k2, XR0 = (0.5 * r) * k0, XR2 = -r * (q2 - 0.5 * k2);
+  double vb = bLX[2] * (XL0 + XL2) + bRX[2] * (XR0 + XR2);
+  double s1b = bLX[1] * XL0 + bRX[1] * XR0, s3b = bLX[1] * XL2 + bRX[1] * XR2;
+  const double oL = bLX[0] + bLX[2] * w.v, oR = bRX[0] + bRX[2] * w.v;
+  const double XLb0 = oL + bLX[1] * w.s1, XLb1 = bLX[2], XLb2 = oL + bLX[1] * w.s3;
+  const double XRb0 = oR + bRX[1] * w.s1, XRb1 = bRX[2], XRb2 = oR + bRX[1] * w.s3;
+  // ---- transverse: down-going along v - a (and v < 0), up-going along v + a (and v > 0)
+  const double wt = -0.5 * r * rt, g0 = w.v - w.a, g2 = w.v + w.a;
+  const double wm0 = wt * g0, wp2 = wt * g2, wm1 = w.v < 0.0 ? wt * w.v : 0.0, wp1 = w.v > 0.0 ? wt * w.v : 0.0;
+  double ub = 0.0, ab = 0.0, hab = 0.0, g0b = 0.0, g2b = 0.0, wm0b = 0.0, w1mb = 0.0, w1pb = 0.0, wp2b = 0.0;
+  double Ab0, Ab1, Ab2, Bb0, Bb1, Bb2;
+  auto trans = [&](double V0, double V1, double V2, const double* om, const double* op, double& Vb0, double& Vb1,
+                   double& Vb2) {
+    const double m = 0.5 * (V0 + V2), d = V1 * w.ha, dV = V2 - V0;
+    const double b0 = m - d, b1 = w.a * dV, b2 = m + d;
+    const double x0 = wm0 * b0, x2 = wp2 * b2;
+    ub += om[1] * x0 + op[1] * x2;
+    g0b += om[2] * x0;
+    g2b += op[2] * x2;
+    const double cm = (om[0] + om[1] * w.u) + om[2] * g0, cp = (op[0] + op[1] * w.u) + op[2] * g2;
+    wm0b += cm * b0;
+    wp2b += cp * b2;
+    w1mb += om[1] * b1;
+    w1pb += op[1] * b1;
+    const double bb0 = cm * wm0, bb1 = om[1] * wm1 + op[1] * wp1, bb2 = cp * wp2;
+    const double hm = 0.5 * (bb0 + bb2), db = bb2 - bb0, t = bb1 * w.a;
+    ab += bb1 * dV;
+    hab += db * V1;
+    Vb0 = hm - t;
+    Vb1 = db * w.ha;
+    Vb2 = hm + t;
+  };
+  trans(A0, A1, A2, bLG1, bLG2, Ab0, Ab1, Ab2);
+  trans(B0, B1, B2, bRG1, bRG2, Bb0, Bb1, Bb2);
+  g0b += wm0b * wt;
+  g2b += wp2b * wt;
+  vb += g0b + g2b + (w.v < 0.0 ? w1mb : (w.v > 0.0 ? w1pb : 0.0)) * wt;
+  ab += g2b - g0b;
+  // ---- e, q, k of each wave
+  const double hr = 0.5 * r;
+  const double eb0 = Ab0 - r * XLb0, eb1 = Ab1 - r * XLb1, qb1 = Bb1 - r * XRb1, qb2 = Bb2 - r * XRb2;
+  const double kb0 = hr * (XRb0 - XLb0) + (Ab0 - Bb0), kb1 = hr * (XRb1 - XLb1) + (Ab1 - Bb1),
+               kb2 = hr * (XRb2 - XLb2) + (Ab2 - Bb2);
+  // ---- limiter
+  const double t0b = kb0 * c0 * dt0, t1b = kb1 * c1 * dt1, t2b = kb2 * c2 * dt2;
+  const double x1 = uneg ? eb1 : qb1;
+  const double sab1 = kb1 * p1 * (1.0 - 2.0 * r * au);
+  const double a1b = kb0 * c0 * da0 + eb0 * w.s1, a2b = kb1 * c1 * da1 + x1 * w.u, a3b = kb2 * c2 * da2 + qb2 * w.s3;
+  s1b += eb0 * w.a1 - kb0 * p0 * (1.0 + 2.0 * r * w.s1);
+  ub += x1 * w.a2 + (uneg ? -sab1 : sab1);
+  s3b += qb2 * w.a3 + kb2 * p2 * (1.0 - 2.0 * r * w.s3);
+  const double U0b = t0b * in0, U2b = t2b * in2;
+  const double mr0b = U0b * nr.a1, ml2b = U2b * nl.a3;
+  NRb.a1 = U0b * mr0;
+  NRb.a2 = right ? 0.0 : t1b;
+  NRb.s1 = mr0b * w.s1;
+  NRb.v = mr0b * w.v;
+  NLb.a3 = U2b * ml2;
+  NLb.a2 = right ? t1b : 0.0;
+  NLb.s3 = ml2b * w.s3;
+  NLb.v = ml2b * w.v;
+  const double n1b = -2.0 * (t0b * U0) * (in0 * in0), n3b = -2.0 * (t2b * U2) * (in2 * in2);
+  Wb.a1 = a1b;
+  Wb.a2 = a2b;
+  Wb.a3 = a3b;
+  Wb.u = ub;
+  Wb.v = vb + w.v * (n1b + n3b) + ml2b * nl.v + mr0b * nr.v;
+  Wb.a = ab;
+  Wb.ha = hab;
+  Wb.s1 = s1b + w.s1 * n1b + mr0b * nr.s1;
+  Wb.s3 = s3b + w.s3 * n3b + ml2b * nl.s3;
+}
+#endif
 
 // One interface with its four input cells A = k-2, L = k-1, R = k, B = k+1 (frame vectors):
 // accumulates the adjoints of the four cells (frame) into gA..gB.
