@@ -1308,44 +1308,46 @@ static int fit_wpb(const claw2d_desc* d, long items, int most) {
 // occupancy cache index of a wavefronts-per-workgroup count 1, 2 or 4
 static int wpb_index(int wpb) { return wpb == 1 ? 0 : (wpb == 2 ? 1 : 2); }
 
-// Rows per marching segment.  A wavefront's run time is proportional to its rows, so the grid
-// is cut into as many segments as fit in one resident round (every wavefront starts at once
-// and ends at once), of at least 16 rows: each segment re-solves 4 halo rows.  A small grid whose
-// 16-row segments would leave more than half the SIMDs idle runs latency-bound, one wavefront per
-// SIMD, where time follows the rows per wavefront; it is cut for half the SIMDs instead, down to
-// 4 rows (FP64 shallow water, 256^2: 43.3 -> 27.4 us per step; 512^2: 45.2 -> 40.1 us).  An
-// explicit desc->seg_h overrides this.
-static int choose_seg_h(const claw2d_desc* d, long resident) {
+// Rows per marching segment.  A wavefront's run time is proportional to its rows (4 of them halo
+// rows that each segment solves again), and every wavefront of a launch starts at once where the
+// kernel's occupancy allows it.  So the grid is cut for w wavefronts per SIMD, w = 1/2, 1, 2 .. the
+// occupancy, and the w of the least estimated time is taken.  A row of w wavefronts that share a SIMD
+// takes rel(w) times the row of one (FP64 is close to its issue limit with one; FP32 and long rows
+// gain more from a second), a segment costs about 6 rows beside its own (halo rows, launch, the
+// pipeline's start), and filling more than half the SIMDs about 2 more (arrivals, doubled CUs).
+// Fewer wavefronts win a tie.  Measured on MI355X, before (whole rounds of at least 16 rows, or half
+// the SIMDs and 4 rows) -> now, FP64 shallow water: 64^2 16.9 -> 13.6 us, 400^2 21.6 -> 18.0,
+// 512^2 25.7 -> 20.6, 768^2 33 -> 26.6; FP32 768^2 31 -> 21.8; FP64 Euler 512^2 35 -> 28.4, 1023 x 777
+// 48.8 -> 43.4; from 1500^2 up the segments are the same as before within a row or two.
+// An explicit desc->seg_h overrides this.
+static int choose_seg_h(const claw2d_desc* d, long resident, bool split) {
   if (d->seg_h > 0) return d->seg_h;
-  const long nstrips = (d->mx + kOwn - 1) / kOwn;
-  long nsegs = resident > 0 ? resident / nstrips : 32;
-  long min_rows = 16;
-  const long simds = device_simds(), half = simds / 2;
-  if (nstrips * (((long)d->my + min_rows - 1) / min_rows) < half) {
-    nsegs = half / nstrips;
-    min_rows = 4;
+  const long nstrips = (d->mx + kOwn - 1) / kOwn, my = d->my;
+  const long simds = device_simds();
+  if (resident <= 0 || simds <= 0) return (int)((my + 31) / 32);
+  bool same = true;
+  for (int p = 1; p < d->num_waves; ++p) same = same && d->mthlim[p] == d->mthlim[0];
+  const bool fast = same && (d->mthlim[0] == 1 || d->mthlim[0] == 4);  // a limiter with kernels of its own
+  const bool long_rows = d->solver == CLAW_SOLVER_EULER_4WAVE || !fast;
+  static const double kRel64[4] = {1.0, 1.65, 2.3, 3.0}, kRel64Long[4] = {1.0, 1.45, 2.1, 2.8};
+  static const double kRel64Split[4] = {1.0, 1.5, 2.15, 2.8}, kRel32[4] = {1.0, 1.22, 1.55, 2.0};
+  const double* rel = d->dtype != CLAW_FP64 ? kRel32 : (long_rows ? kRel64Long : (split ? kRel64Split : kRel64));
+  const long most = std::min(4L, std::max(1L, resident / simds));
+  long best_h = my;
+  double best = 1e300;
+  for (long w = 0; w <= most; ++w) {  // 0 stands for half a wavefront per SIMD
+    const long nsegs = (w == 0 ? simds / 2 : w * simds) / nstrips;
+    if (nsegs < 1) continue;
+    const long h = (my + nsegs - 1) / nsegs;
+    const double t = (w > 0 ? rel[w - 1] : 1.0) * (double)(h + 6) + (w > 0 ? 2.0 : 0.0);
+    if (t < best) {
+      best = t;
+      best_h = h;
+    }
   }
-  nsegs = std::max(1L, std::min(nsegs, ((long)d->my + min_rows - 1) / min_rows));
-  // More than 2 wavefronts per SIMD in segments under 32 rows re-solve more halo rows than the
-  // extra occupancy returns: cut for 2 per SIMD instead.  At 2048^2 (18-row segments at 4 per
-  // SIMD -> 36 rows at 2): shallow water FP32 135.9 -> 114.3 us, split 131.3 -> 107.1 us;
-  // bathymetry FP32 138.1 -> 108.9 us, split 132.4 -> 101.7 us; FP64 split (24 rows at 3 per SIMD)
-  // 128.4 -> 122.5 us.  The Euler kernels keep the occupancy sizing: FP32 135.2 -> 139.2 us there.
-  long seg0 = ((long)d->my + nsegs - 1) / nsegs;
-  long waves = nstrips * (((long)d->my + seg0 - 1) / seg0);
-  if (simds > 0 && d->solver != CLAW_SOLVER_EULER_4WAVE && waves > 2 * simds && seg0 < 32) {
-    nsegs = std::max(1L, 2 * simds / nstrips);
-    seg0 = ((long)d->my + nsegs - 1) / nsegs;
-    waves = nstrips * (((long)d->my + seg0 - 1) / seg0);
-  }
-  // A launch just over a whole number m of wavefronts per SIMD (by up to a quarter of the SIMDs)
-  // leaves those few SIMDs a round more than the rest, and they set the time; it is cut to m
-  // per SIMD instead (FP64 shallow water 1024^2: 1152 wavefronts 81.2 us, 936 wavefronts 66.9 us).
-  if (simds > 0 && waves > simds) {
-    const long m = waves / simds;
-    if (waves - m * simds <= simds / 4 && m * simds / nstrips >= 1) nsegs = m * simds / nstrips;
-  }
-  return (int)((d->my + nsegs - 1) / nsegs);
+  // (strips alone fill the device: whole columns, or 64 rows where that leaves a poor last round)
+  if (best == 1e300) best_h = std::min(my, 64L);
+  return (int)best_h;
 }
 
 static int check_desc(const claw2d_desc* d) {
@@ -1401,14 +1403,14 @@ static int check_desc(const claw2d_desc* d) {
 }
 
 template <class T, class P>
-static void fill_args(StepArgs<T, P>& a, const claw2d_desc* d, long resident) {
+static void fill_args(StepArgs<T, P>& a, const claw2d_desc* d, long resident, bool split) {
   a.wpb = launch_wpb(d);
   a.xcd = d->launch_order == 0 ? 1 : 0;
   a.dx = d->dx;
   a.dy = d->dy;
   a.mx = d->mx;
   a.my = d->my;
-  a.seg_h = choose_seg_h(d, resident);
+  a.seg_h = choose_seg_h(d, resident, split);
   a.nstrips = (d->mx + kOwn - 1) / kOwn;
   a.nsegs = (d->my + a.seg_h - 1) / a.seg_h;
   a.bcx_lo = d->bc_lower[0];
@@ -1496,7 +1498,7 @@ static int launch_step(const claw2d_desc* d, const typename P::Par& par, void* q
   long& res = cached[slot][wpb_index(launch_wpb(d))];
   if (res < 0) res = resident_waves(kern, launch_wpb(d));
   StepArgs<T, P> a;
-  fill_args(a, d, res);
+  fill_args(a, d, res, SPLIT);
   a.q0 = (T*)q0;
   a.q1 = (T*)q1;
   a.ctrl = ctrl;
@@ -1533,7 +1535,7 @@ static int launch_sweep(const claw2d_desc* d, const typename P::Par& par, const 
   long& res = cached[ids - 1][wpb_index(wpb)];
   if (res < 0) res = resident_waves(kern, wpb);
   StepArgs<T, P> a;
-  fill_args(a, d, res);
+  fill_args(a, d, res, true);
   a.q0 = (T*)qbc;
   a.q1 = (T*)qout;
   a.ctrl = ctrl;
@@ -1613,7 +1615,7 @@ static int launch_batch(const claw2d_desc* d, const typename P::Par& par, const 
   static thread_local long cached[5] = {-1, -1, -1, -1, -1};
   if (cached[slot] < 0) cached[slot] = resident_waves(kern);
   StepArgs<T, P> a;
-  fill_args(a, d, cached[slot]);
+  fill_args(a, d, cached[slot], false);
   a.q0 = (T*)q0;
   a.q1 = (T*)q1;
   a.ctrl = nullptr;
