@@ -3,8 +3,8 @@
 All grids share the method (solver, precision, limiters, BCs, physics) and differ in size and
 spacing; each keeps its own time, its own CFL-chosen dt and its own accept/reject history, as if
 each had its own pyclaw solver.  Per attempt the library launches one persistent kernel over the
-(grid, strip, segment) work items of every grid plus one per-grid control kernel; a run of
-attempts can be captured once as a HIP graph and replayed.
+(grid, strip, segment) work items of every grid; the last item of a grid to finish applies its
+accept/reject and dt.  A run of attempts can be captured once as a HIP graph and replayed.
 """
 import ctypes as C
 

@@ -1075,8 +1075,13 @@ step2_fused(StepArgs<T, P> a) {
 
 // Batched grids: every grid's planes live in one ping-pong pair at its own offset, each grid has
 // its own control block (its own CFL-chosen dt), and a persistent set of wavefronts takes
-// (grid, strip, segment) work items from an atomic counter.  The counter is reset by the batch
-// control kernel, so a captured sequence of launches contains no memset.
+// (grid, strip, segment) work items: its first by its own number, the rest from an atomic counter
+// (one ticket per item from every wavefront at the start was 1900 device-scope atomics on one line).
+// The last item of a grid to finish runs its controller, as the last workgroup of a single-grid step
+// does, so an attempt is one launch; a second launch with one thread per grid took 5 us and its gap.
+// Every item is followed by one ticket, so the last ticket of a launch is known and resets the
+// counter: a captured sequence of launches contains no memset.
+// 64 grids of 64^2 to 512^2, an attempt: 169 -> 132 us with this and batch_rows' cut.
 struct BatchDev {
   const claw2d_batch_grid* grids;
   claw2d_ctrl* ctrls;
@@ -1085,50 +1090,56 @@ struct BatchDev {
   int total_items;
 };
 
+// The last grid whose item0 <= item (item0 ascends from 0): 64 grids are probed at once, one per lane.
+__device__ __forceinline__ int grid_of_item(const BatchDev& b, int item) {
+  const int lane = threadIdx.x & 63;
+  int lo = 0, n = b.ngrids;  // the grid is one of lo .. lo + n - 1
+  while (n > 1) {
+    const int stride = (n + 63) >> 6, k = lane * stride;
+    const unsigned long long le = lanes(k < n && b.grids[lo + (k < n ? k : 0)].item0 <= item);
+    const int j = 63 - __builtin_clzll(le);  // lane 0 always holds; lanes that hold are 0 .. j
+    lo += j * stride;
+    n = min(stride, n - j * stride);
+  }
+  return __builtin_amdgcn_readfirstlane(lo);
+}
+
 template <class T, class P, int LIM, int TWC>
 __global__ void __launch_bounds__(kLanes* kWPB) __attribute__((amdgpu_waves_per_eu(MinWaves<T>::value)))
 batch_step(StepArgs<T, P> a, BatchDev b) {
   const int lane = threadIdx.x & 63;
-  for (;;) {
-    // every lane takes part (lane 0 adds 1, the others 0) and lane 0's ticket is broadcast, so
-    // no lane-divergent region sits inside this loop
-    const int item = __builtin_amdgcn_readfirstlane(atomicAdd(b.counter, lane == 0 ? 1 : 0));
-    if (item >= b.total_items) break;
-    int lo = 0, hi = b.ngrids - 1;  // last grid whose item0 <= item
-    while (lo < hi) {
-      const int mid = (lo + hi + 1) >> 1;
-      if (b.grids[mid].item0 <= item) lo = mid;
-      else hi = mid - 1;
-    }
-    const int gi = __builtin_amdgcn_readfirstlane(lo);
+  const int first = (int)gridDim.x * kWPB;  // items taken by number
+  int item = __builtin_amdgcn_readfirstlane(xcd_remap(blockIdx.x, gridDim.x) * kWPB + (threadIdx.x >> 6));
+  // no lane-divergent region sits inside this loop (every lane takes part in the tickets: lane 0 adds
+  // 1, the others 0; every lane runs the controller, all with the same values)
+  while (item < b.total_items) {
+    const int gi = grid_of_item(b, item);
     const claw2d_batch_grid& G = b.grids[gi];
     claw2d_ctrl* c = b.ctrls + gi;
-    if (c->done) continue;
-    const double dt = c->dt;
-    const T* qin = (c->cur ? a.q1 : a.q0) + G.offset;
-    T* qout = (c->cur ? a.q0 : a.q1) + G.offset;
-    const int local = item - G.item0;
-    const int strip = local % G.nstrips, seg = local / G.nstrips;
-    const int x0 = strip * kOwn, y0 = seg * G.seg_h;
-    const int y1 = min(y0 + G.seg_h, G.my);
-    publish_max(c, march_item<T, P, LIM, false, TWC>(a, qin, qout, G.mx, G.my, x0, y0, y1, dt, G.dx, G.dy), false);
+    if (!c->done) {
+      const double dt = c->dt;
+      const T* qin = (c->cur ? a.q1 : a.q0) + G.offset;
+      T* qout = (c->cur ? a.q0 : a.q1) + G.offset;
+      const int local = item - G.item0;
+      const int strip = local % G.nstrips, seg = local / G.nstrips;
+      const int x0 = strip * kOwn, y0 = seg * G.seg_h;
+      const int y1 = min(y0 + G.seg_h, G.my);
+      publish_max(c, march_item<T, P, LIM, false, TWC>(a, qin, qout, G.mx, G.my, x0, y0, y1, dt, G.dx, G.dy), false);
+      // the maxima are performed before the arrival (see step2_fused)
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      const int arrived = __builtin_amdgcn_readfirstlane(atomicAdd(&c->arrive, lane == 0 ? 1 : 0));
+      if (arrived == G.nstrips * G.nsegs - 1) {
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+        control_one(c, G.dx, G.dy, a.cfl_max, a.cfl_desired, a.dt_max);
+        c->arrive = 0;
+      }
+    }
+    if (b.total_items <= first) break;  // one item each
+    const int ticket = __builtin_amdgcn_readfirstlane(atomicAdd(b.counter, lane == 0 ? 1 : 0));
+    if (ticket == b.total_items - 1) *b.counter = 0;
+    item = first + ticket;
   }
 }
-
-
-// One evolve_to_time iteration after the step (upstream pyclaw solver.py): accept/reject,
-// advance t, choose the next dt, clip it to tend.
-
-#ifndef CLAW_KERNEL_UNIT
-// One thread per grid; thread 0 also rearms the work counter of the batched step.
-__global__ void batch_control(const claw2d_batch_grid* grids, claw2d_ctrl* ctrls, int* counter,
-                              int ngrids, double cfl_max, double cfl_desired, double dt_max) {
-  const int g = blockIdx.x * blockDim.x + threadIdx.x;
-  if (g == 0) *counter = 0;
-  if (g >= ngrids) return;
-  control_one(ctrls + g, grids[g].dx, grids[g].dy, cfl_max, cfl_desired, dt_max);
-}
-#endif
 
 // ------------------------------------------------------------------------------------------
 // Compensated FP64 sum of one component, fixed reduction order.
@@ -1308,13 +1319,26 @@ static int fit_wpb(const claw2d_desc* d, long items, int most) {
 // occupancy cache index of a wavefronts-per-workgroup count 1, 2 or 4
 static int wpb_index(int wpb) { return wpb == 1 ? 0 : (wpb == 2 ? 1 : 2); }
 
+// Time of a marched row of w = 1 .. 4 wavefronts that share a SIMD, relative to the row of one alone
+// (measured on MI355X: FP64 is close to its issue limit with one; FP32 and the long rows of Euler and
+// of the general limiter kernel gain more from a second).
+static const double* row_times(const claw2d_desc* d, bool split) {
+  static const double kRel64[4] = {1.0, 1.65, 2.3, 3.0}, kRel64Long[4] = {1.0, 1.45, 2.1, 2.8};
+  static const double kRel64Split[4] = {1.0, 1.5, 2.15, 2.8}, kRel32[4] = {1.0, 1.22, 1.55, 2.0};
+  bool same = true;
+  for (int p = 1; p < d->num_waves; ++p) same = same && d->mthlim[p] == d->mthlim[0];
+  const bool own = same && (d->mthlim[0] == 1 || d->mthlim[0] == 4);  // a limiter with kernels of its own
+  if (d->dtype != CLAW_FP64) return kRel32;
+  if (d->solver == CLAW_SOLVER_EULER_4WAVE || !own) return kRel64Long;
+  return split ? kRel64Split : kRel64;
+}
+
 // Rows per marching segment.  A wavefront's run time is proportional to its rows (4 of them halo
 // rows that each segment solves again), and every wavefront of a launch starts at once where the
 // kernel's occupancy allows it.  So the grid is cut for w wavefronts per SIMD, w = 1/2, 1, 2 .. the
 // occupancy, and the w of the least estimated time is taken.  A row of w wavefronts that share a SIMD
-// takes rel(w) times the row of one (FP64 is close to its issue limit with one; FP32 and long rows
-// gain more from a second), a segment costs about 6 rows beside its own (halo rows, launch, the
-// pipeline's start), and filling more than half the SIMDs about 2 more (arrivals, doubled CUs).
+// takes row_times' share, a segment costs about 6 rows beside its own (halo rows, launch, the pipeline's
+// start), and filling more than half the SIMDs about 2 more (arrivals).
 // Fewer wavefronts win a tie.  Measured on MI355X, before (whole rounds of at least 16 rows, or half
 // the SIMDs and 4 rows) -> now, FP64 shallow water: 64^2 16.9 -> 13.6 us, 400^2 21.6 -> 18.0,
 // 512^2 25.7 -> 20.6, 768^2 33 -> 26.6; FP32 768^2 31 -> 21.8; FP64 Euler 512^2 35 -> 28.4, 1023 x 777
@@ -1325,13 +1349,7 @@ static int choose_seg_h(const claw2d_desc* d, long resident, bool split) {
   const long nstrips = (d->mx + kOwn - 1) / kOwn, my = d->my;
   const long simds = device_simds();
   if (resident <= 0 || simds <= 0) return (int)((my + 31) / 32);
-  bool same = true;
-  for (int p = 1; p < d->num_waves; ++p) same = same && d->mthlim[p] == d->mthlim[0];
-  const bool fast = same && (d->mthlim[0] == 1 || d->mthlim[0] == 4);  // a limiter with kernels of its own
-  const bool long_rows = d->solver == CLAW_SOLVER_EULER_4WAVE || !fast;
-  static const double kRel64[4] = {1.0, 1.65, 2.3, 3.0}, kRel64Long[4] = {1.0, 1.45, 2.1, 2.8};
-  static const double kRel64Split[4] = {1.0, 1.5, 2.15, 2.8}, kRel32[4] = {1.0, 1.22, 1.55, 2.0};
-  const double* rel = d->dtype != CLAW_FP64 ? kRel32 : (long_rows ? kRel64Long : (split ? kRel64Split : kRel64));
+  const double* rel = row_times(d, split);
   const long most = std::min(4L, std::max(1L, resident / simds));
   long best_h = my;
   double best = 1e300;
@@ -1606,16 +1624,23 @@ static const void* batch_kernel(const claw2d_desc* d, int* slot) {
   return (const void*)batch_step<T, P, 0, -1>;
 }
 
+// The batched kernel of a method and its resident wavefronts on the current device.
+template <class T, class P> static long batch_resident(const claw2d_desc* d, const void** kern) {
+  int slot = 0;
+  *kern = batch_kernel<T, P>(d, &slot);
+  static thread_local long cached[5] = {-1, -1, -1, -1, -1};
+  if (cached[slot] < 0) cached[slot] = resident_waves(*kern);
+  return cached[slot];
+}
+
 template <class T, class P>
 static int launch_batch(const claw2d_desc* d, const typename P::Par& par, const claw2d_batch_grid* grids,
                         int ngrids, int total_items, void* q0, void* q1, claw2d_ctrl* ctrls,
                         int32_t* counter, hipStream_t s) {
-  int slot = 0;
-  const void* kern = batch_kernel<T, P>(d, &slot);
-  static thread_local long cached[5] = {-1, -1, -1, -1, -1};
-  if (cached[slot] < 0) cached[slot] = resident_waves(kern);
+  const void* kern = nullptr;
+  const long resident = batch_resident<T, P>(d, &kern);
   StepArgs<T, P> a;
-  fill_args(a, d, cached[slot], false);
+  fill_args(a, d, resident, false);
   a.q0 = (T*)q0;
   a.q1 = (T*)q1;
   a.ctrl = nullptr;
@@ -1623,7 +1648,9 @@ static int launch_batch(const claw2d_desc* d, const typename P::Par& par, const 
   a.dt_fixed = 0.0;
   a.fuse = 0;
   a.total_waves = 0;
-  a.cfl_max = a.cfl_desired = a.dt_max = 0.0;
+  a.cfl_max = d->cfl_max;
+  a.cfl_desired = d->cfl_desired;
+  a.dt_max = d->dt_max;
   a.par = par;
   BatchDev b;
   b.grids = grids;
@@ -1631,12 +1658,56 @@ static int launch_batch(const claw2d_desc* d, const typename P::Par& par, const 
   b.counter = counter;
   b.ngrids = ngrids;
   b.total_items = total_items;
-  const long res = cached[slot] > 0 ? cached[slot] : 4096;
+  const long res = resident > 0 ? resident : 4096;
   const long waves = std::min<long>(total_items, res);
   const int blocks = (int)((waves + kWPB - 1) / kWPB);
   void* args[] = {&a, &b};
   const hipError_t e = hipLaunchKernel(kern, dim3(blocks), dim3(kLanes * kWPB), args, 0, s);
   return e == hipSuccess ? 0 : hip_fail(e, "batch_step launch");
+}
+
+// Resident wavefronts of the batched kernel for a method, 0 without a device.
+static long batch_slots(const claw2d_desc* d) {
+  const bool swe = d->solver == CLAW_SOLVER_SHALLOW_ROE_EFIX;
+  const void* k = nullptr;
+  if (device_simds() <= 0) return 0;
+  if (d->dtype == CLAW_FP64) return swe ? batch_resident<double, SweP<double>>(d, &k) : batch_resident<double, EulerP<double>>(d, &k);
+  return swe ? batch_resident<float, SweP<float>>(d, &k) : batch_resident<float, EulerP<float>>(d, &k);
+}
+
+// Rows per segment of a batch, an upper bound: each grid is cut evenly into segments of at most this
+// many.  Where all items run at once (w wavefronts per SIMD) the attempt takes one item's time, as in
+// choose_seg_h; where there are more than the device holds, the items' total over the device plus
+// half an item for the uneven end.  (Segments of 64 rows with a short last one, whatever the grids,
+// had made the longest item 68 rows where the mean was 52.)
+static int batch_rows(const claw2d_desc* d, const claw2d_batch_grid* grids, int ngrids) {
+  const long simds = device_simds(), slots = batch_slots(d);
+  int most_rows = 1;
+  for (int g = 0; g < ngrids; ++g) most_rows = std::max(most_rows, (int)grids[g].my);
+  if (simds <= 0 || slots < simds) return std::max(16, std::min(64, most_rows));
+  const double* rel = row_times(d, false);
+  const long most = std::min(4L, slots / simds);
+  int best_h = 64;
+  double best = 1e300;
+  for (int h = 2; h <= std::min(most_rows, 256); ++h) {
+    long items = 0;
+    double rows = 0.0;  // with the 6 rows' worth of a segment's own cost
+    int longest = 0;
+    for (int g = 0; g < ngrids; ++g) {
+      const long ns = (grids[g].mx + kOwn - 1) / kOwn, k = (grids[g].my + h - 1) / h;
+      items += ns * k;
+      rows += (double)ns * (double)(grids[g].my + 6 * k);
+      longest = std::max(longest, (int)((grids[g].my + k - 1) / k));
+    }
+    const long w = (items + simds - 1) / simds;
+    const double t = w <= most ? rel[w - 1] * (longest + 6) + (2 * items > simds ? 2.0 : 0.0)
+                               : rel[most - 1] * (rows / (double)(most * simds) + 0.5 * (longest + 6));
+    if (t < best) {
+      best = t;
+      best_h = h;
+    }
+  }
+  return best_h;
 }
 
 static int batch_attempt(const claw2d_desc* d, const claw2d_batch_grid* grids, int ngrids,
@@ -1650,12 +1721,7 @@ static int batch_attempt(const claw2d_desc* d, const claw2d_batch_grid* grids, i
   else
     rc = swe ? launch_batch<float, SweP<float>>(d, swe_par<float>(d), grids, ngrids, total_items, q0, q1, ctrls, counter, s)
              : launch_batch<float, EulerP<float>>(d, euler_par<float>(d), grids, ngrids, total_items, q0, q1, ctrls, counter, s);
-  if (rc) return rc;
-  const int threads = 256, blocks = (ngrids + threads - 1) / threads;
-  hipLaunchKernelGGL(batch_control, dim3(blocks), dim3(threads), 0, s, grids, ctrls, (int*)counter,
-                     ngrids, d->cfl_max, d->cfl_desired, d->dt_max);
-  const hipError_t e = hipGetLastError();
-  return e == hipSuccess ? 0 : hip_fail(e, "batch_control launch");
+  return rc;
 }
 
 static int check_batch(const claw2d_desc* d, const void* grids, int32_t ngrids, int64_t total_items,
@@ -1930,12 +1996,15 @@ int claw2d_batch_prepare(const claw2d_desc* d, claw2d_batch_grid* grids, int32_t
   if (ngrids < 1) return fail(-30, "ngrids must be >= 1");
   if (seg_h < 0) return fail(-14, "seg_h must be >= 0");
   long long items = 0;
+  for (int g = 0; g < ngrids; ++g)
+    if (grids[g].mx < 2 || grids[g].my < 2) return fail(-5, "every grid needs mx, my >= 2");
+  const int rows = seg_h > 0 ? seg_h : batch_rows(d, grids, ngrids);
   for (int g = 0; g < ngrids; ++g) {
     claw2d_batch_grid& G = grids[g];
-    if (G.mx < 2 || G.my < 2) return fail(-5, "every grid needs mx, my >= 2");
     if (!(G.dx > 0) || !(G.dy > 0)) return fail(-13, "dx, dy must be positive");
     if (G.offset < 0) return fail(-32, "negative grid offset");
-    const int h = seg_h > 0 ? seg_h : std::max(16, std::min(64, (int)G.my));
+    const int k = (G.my + rows - 1) / rows;
+    const int h = seg_h > 0 ? seg_h : (G.my + k - 1) / k;
     G.seg_h = h;
     G.nstrips = (G.mx + kOwn - 1) / kOwn;
     G.nsegs = (G.my + h - 1) / h;

@@ -259,9 +259,9 @@ int claw2d_batch_prepare(const claw2d_desc* d, claw2d_batch_grid* grids, int32_t
                          int32_t seg_h, int64_t* total_items);
 
 /* Enqueues `attempts` evolve_to_time attempts of every grid: one persistent batched step kernel
- * and one per-grid control kernel per attempt.  grids_dev is the prepared table copied to the
+ * per attempt, in which the last item of a grid to finish applies the grid's accept/reject and dt.  grids_dev is the prepared table copied to the
  * device; ctrls_dev holds ngrids control blocks; counter_dev is one int, zero before the first
- * call (the control kernel rearms it). */
+ * call (each attempt leaves it zero). */
 int claw2d_batch_advance(const claw2d_desc* d, const claw2d_batch_grid* grids_dev, int32_t ngrids,
                          int64_t total_items, void* q0_dev, void* q1_dev, claw2d_ctrl* ctrls_dev,
                          int32_t* counter_dev, long long attempts, void* stream);
