@@ -171,7 +171,7 @@ template <class T, class P> struct StepArgs {
   int mx, my, nstrips, nsegs, seg_h;
   int bcx_lo, bcx_hi, bcy_lo, bcy_hi, rfx, rfy;
   int order, tw;
-  int mthlim[4];
+  int mthlim[4], lim_all;  // lim_all: the id all waves share, or -1
   // 0: no controller; 1: the last wavefront writes the CFL number of the fixed-dt step;
   // 2: the last wavefront runs the evolve_to_time controller on ctrl
   int fuse;
@@ -192,6 +192,30 @@ template <class P, class T>
 __device__ __forceinline__ typename P::Cell prep_cell(const T q[P::NEQ], T b, const typename P::Par& pr) {
   if constexpr (P::NAUX > 0) return P::prep(q, b, pr);
   else return P::prep(q, pr);
+}
+
+// The limited strengths of an interface's waves: t[p] (the upwind term) is replaced by
+// phi(t/alpha) alpha.  LIM 0: ids from a; where all waves have one, it is branched on once per
+// interface and the waves' operations stay in one block.
+template <int LIM, class T, class P, int NW>
+__device__ __forceinline__ void limit_waves(const T (&al)[NW], T (&t)[NW], const StepArgs<T, P>& a) {
+  auto all = [&](auto meth) {
+#pragma unroll
+    for (int p = 0; p < NW; ++p) t[p] = limited(al[p], t[p], decltype(meth)::value);
+  };
+  if constexpr (LIM > 0) {
+    all(std::integral_constant<int, LIM>{});
+  } else {
+    switch (a.lim_all) {
+      case 1: all(std::integral_constant<int, 1>{}); break;
+      case 2: all(std::integral_constant<int, 2>{}); break;
+      case 3: all(std::integral_constant<int, 3>{}); break;
+      case 4: all(std::integral_constant<int, 4>{}); break;
+      default:
+#pragma unroll
+        for (int p = 0; p < NW; ++p) t[p] = limited(al[p], t[p], a.mthlim[p]);
+    }
+  }
 }
 
 // Limits one interface and forms its contributions (interface frame), following flux2.f90:
@@ -228,19 +252,24 @@ __device__ __forceinline__ void finish_iface(const typename P::Iface& f, const T
   T in[NW];
   if (second) P::inv_norm(f, in);
   const T rc = CAPA ? T(0.5) * (r * rkL + r * rkR) : r;  // dt/dx of the correction
-  T XL[NW], XR[NW], A[NW], B[NW];
+  T XL[NW], XR[NW], A[NW], B[NW], lt[NW];
+  if (second) {
+#pragma unroll
+    for (int p = 0; p < NW; ++p) {
+      const T aL = upL[p], aR = alR[p], mr = mR[p];  // rvalues: no lvalue select
+      lt[p] = (P::speed(f, p) > T(0) ? aL : aR * mr) * in[p];
+    }
+    limit_waves<LIM>(f.al, lt, a);
+  }
 #pragma unroll
   for (int p = 0; p < NW; ++p) {
     const T s = P::speed(f, p), al = f.al[p], sf = sfs[p];
     const T e = sf * al, q = P::FWAVE ? al - e : (s - sf) * al;
     T k = T(0);
     if (second) {
-      const T aL = upL[p], aR = alR[p], mr = mR[p];  // rvalues: no lvalue select
-      const T t = (s > T(0) ? aL : aR * mr) * in[p];
-      const int meth = LIM > 0 ? LIM : a.mthlim[p];
       const T sa = vabs(s);  // |s| as a source modifier (a select form costs two instructions)
       const T sw = P::FWAVE ? copysign(T(1), s) : sa;
-      k = sw * (T(1) - sa * rc) * limited(al, t, meth);
+      k = sw * (T(1) - sa * rc) * lt[p];
     }
     XL[p] = -r * fma(T(0.5), k, e);
     XR[p] = -r * fma(T(-0.5), k, q);
@@ -305,22 +334,27 @@ __device__ __forceinline__ void finish_plain(const typename P::Iface& f, const T
   T in[NW];
   if (second) P::inv_norm(f, in);
   const T rc = CAPA ? T(0.5) * (r * rkL + r * rkR) : r;
-  T XL[NW], XR[NW], A[NW], B[NW];
+  T XL[NW], XR[NW], A[NW], B[NW], lt[NW];
+  if (second) {
+#pragma unroll
+    for (int p = 0; p < NW; ++p) {
+      const int side = P::side(p);
+      const T aR = alR[p], mr = mR[p];
+      if (side < 0) lt[p] = (aR * mr) * in[p];
+      else if (side > 0) lt[p] = upL[p] * in[p];
+      else lt[p] = (P::speed(f, p) > T(0) ? upL[p] : aR * mr) * in[p];
+    }
+    limit_waves<LIM>(f.al, lt, a);
+  }
 #pragma unroll
   for (int p = 0; p < NW; ++p) {
     const int side = P::side(p);
     const T s = P::speed(f, p), al = f.al[p];
     T k = T(0);
     if (second) {
-      const T aR = alR[p], mr = mR[p];
-      T t;
-      if (side < 0) t = (aR * mr) * in[p];
-      else if (side > 0) t = upL[p] * in[p];
-      else t = (s > T(0) ? upL[p] : aR * mr) * in[p];
-      const int meth = LIM > 0 ? LIM : a.mthlim[p];
       const T sa = side < 0 ? -s : (side > 0 ? s : vabs(s));
       const T sw = P::FWAVE ? (side < 0 ? T(-1) : (side > 0 ? T(1) : copysign(T(1), s))) : sa;
-      k = sw * (T(1) - sa * rc) * limited(al, t, meth);
+      k = sw * (T(1) - sa * rc) * lt[p];
     }
     const T hk = T(0.5) * k;
     if (side < 0) {
@@ -1439,7 +1473,11 @@ static void fill_args(StepArgs<T, P>& a, const claw2d_desc* d, long resident, bo
   a.rfy = d->reflect_index[1];
   a.order = d->order;
   a.tw = d->transverse_waves;
-  for (int p = 0; p < 4; ++p) a.mthlim[p] = d->mthlim[p];
+  a.lim_all = d->mthlim[0];
+  for (int p = 0; p < 4; ++p) {
+    a.mthlim[p] = d->mthlim[p];
+    if (p < P::NW && d->mthlim[p] != a.lim_all) a.lim_all = -1;
+  }
   a.aux = nullptr;
   a.capa = nullptr;
   a.abx_lo = d->aux_bc_lower[0];

@@ -96,6 +96,15 @@ __device__ __forceinline__ float flip_sign(float x, float s) {
   return __int_as_float(__float_as_int(x) ^ (__float_as_int(s) & (int)0x80000000u));
 }
 
+// Reciprocal to about half an ulp in both types (the FP32 instruction alone has 1), and the smallest
+// normal operand it takes.
+__device__ __forceinline__ double frcp_near(double x) { return frcp(x); }
+__device__ __forceinline__ float frcp_near(float x) {
+  const float y = frcp(x);
+  return fmaf(y, fmaf(-x, y, 1.0f), y);
+}
+template <class T> constexpr T kTiny = sizeof(T) == 8 ? T(2.3e-308) : T(1.2e-38f);
+
 // phi(t/alpha)*alpha for limiter `meth` (ids of pyclaw/limiters/tvd.py: minmod 1, superbee 2,
 // van Leer 3, MC 4, beam-warming 5, 0 = unlimited).  alpha == 0 gives 0 (upstream skips a wave
 // of zero norm, which is the zero wave).  minmod, superbee and MC are odd in (alpha, t), so they
@@ -110,10 +119,11 @@ template <class T> __device__ __forceinline__ T limited(T al, T t, int meth) {
       const T lo = vmax(vmin_abs(al, T(2) * ts), vmin_abs(T(2) * al, ts));
       return flip_sign(vmax0(lo), al);
     }
-    case 3: {  // van Leer: (theta + |theta|)/(1 + |theta|)
-      if (al == T(0)) return T(0);
-      const T th = t / al, ath = th < T(0) ? -th : th;
-      return al * ((th + ath) / (T(1) + ath));
+    case 3: {  // van Leer: 2 theta/(1 + theta) for theta > 0, so 2 |alpha| ts/(|alpha| + ts): one
+               // reciprocal where theta and phi took two divisions (the clamp keeps it finite):
+               // with one branch per interface (limit_waves) 4096^2 FP64 428 -> 350 us
+      const T a = vabs(al), r = a * frcp_near(vmax(a + ts, T(kTiny<T>)));
+      return ts <= T(0) ? T(0) : flip_sign(r * (T(2) * ts), al);
     }
     case 4: {  // MC: max(0, min((1 + theta)/2, 2, 2 theta))
       const T c = T(0.5) * (vabs(al) + ts);
