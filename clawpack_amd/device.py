@@ -143,11 +143,15 @@ class DeviceGrid:
     def upload(self, q_host):
         """q_host: pyclaw layout (num_eqn, mx, my) -> device planes (num_eqn, my, mx); with a
         depth_ref the depth is stored as h - depth_ref (formed in FP64, then rounded)."""
-        q = torch.from_numpy(np.array(q_host, dtype=np.float64))
+        q = np.asarray(q_host)
+        if q.dtype == np.float64 and q.flags.f_contiguous and q.flags.writeable:
+            # pyclaw's own layout, components fastest: sent as it lies, reordered on the device
+            t = torch.from_numpy(q.T).to(self.device).permute(2, 0, 1)
+        else:
+            t = torch.from_numpy(np.array(q, dtype=np.float64)).permute(0, 2, 1).contiguous().to(self.device)
         if self.desc.depth_ref != 0.0:
-            q[0] -= self.desc.depth_ref
-        planes = q.permute(0, 2, 1).contiguous().to(self.torch_dtype)
-        self.q[self.cur].copy_(planes)
+            t[0] -= self.desc.depth_ref
+        self.q[self.cur].copy_(t)
 
     def set_planes(self, planes):
         """planes: device or host tensor (num_eqn, my, mx)."""
@@ -156,13 +160,21 @@ class DeviceGrid:
     def planes(self):
         return self.q[self.cur]
 
-    def download(self):
+    def download(self, out=None):
         """Current state in pyclaw layout (num_eqn, mx, my), float64 numpy, Fortran order (a
-        stored depth deviation is turned back into h in FP64)."""
-        t = self.q[self.cur].to(torch.float64).cpu()
+        stored depth deviation is turned back into h in FP64).  out: an array of that shape to
+        fill instead of a new one (and to return)."""
+        t = self.q[self.cur].to(torch.float64)
         if self.desc.depth_ref != 0.0:
             t[0] += self.desc.depth_ref
-        return np.asfortranarray(t.permute(0, 2, 1).numpy())
+        t = t.permute(1, 2, 0).contiguous()  # components fastest, reordered on the device
+        if out is None:
+            return t.cpu().numpy().T
+        if out.dtype == np.float64 and out.flags.f_contiguous and out.flags.writeable:
+            torch.from_numpy(out.T).copy_(t)
+        else:
+            out[...] = t.cpu().numpy().T
+        return out
 
     # ---- compute --------------------------------------------------------------------------
     def step(self, dt, stream=None):
