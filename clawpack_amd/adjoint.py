@@ -116,29 +116,31 @@ class FrozenDtEvolve(torch.autograd.Function):
         n = len(dts)
         stepper = _Stepper(desc, q0.device)
         a = q0.detach().contiguous().clone()
-        b = torch.empty_like(a)
-        ckpts = {}
         samples = []
         flat_idx = gauges.to(q0.device)
-        # the states of the last segment are kept as the forward makes them: the backward reverses
-        # that segment first, and would otherwise recompute it from its checkpoint at once
+        # Kept states are stepped into directly, without a copy: the checkpoints, and the states of
+        # the last segment, which the backward reverses first and would otherwise recompute from
+        # its checkpoint at once.  The rest alternate between two scratch states.
         last0 = ((n - 1) // checkpoint_every) * checkpoint_every if n else 0
-        tail = []
+        kept = [k for k in range(1, n) if k % checkpoint_every == 0 or k > last0]
+        store = dict(zip(kept, torch.empty((len(kept),) + tuple(a.shape), dtype=a.dtype, device=a.device)))
+        scratch = [torch.empty_like(a) for _ in range(2)] if len(kept) < n - 1 else []
+        qn = torch.empty_like(a) if n else a
+        store[0] = a
         for k in range(n):
-            if k % checkpoint_every == 0:
-                ckpts[k] = a.clone()
-                if k == last0:
-                    tail.append(ckpts[k])
-            elif k > last0:
-                tail.append(a.clone())
-            stepper.step(a, b, dts[k])
-            a, b = b, a
+            dst = qn if k + 1 == n else store.get(k + 1)
+            if dst is None:
+                dst = scratch[k % 2]
+            stepper.step(a, dst, dts[k])
+            a = dst
             if (k + 1) % sample_every == 0:
                 samples.append(a.view(3, -1)[:, flat_idx])
+        ckpts = {k: store[k] for k in range(0, n, checkpoint_every)}
+        tail = [store[k] for k in range(last0, n)]
         out = torch.stack(samples) if samples else a.new_zeros((0, 3, flat_idx.numel()))
         ctx.desc, ctx.dts, ctx.sample_every, ctx.checkpoint_every = desc, dts, sample_every, checkpoint_every
         ctx.ckpts, ctx.flat_idx, ctx.stepper, ctx.tail = ckpts, flat_idx, stepper, tail
-        return out, a.clone()
+        return out, qn
 
     @staticmethod
     def backward(ctx, g_samples, g_qN):
@@ -179,7 +181,7 @@ class FrozenDtEvolve(torch.autograd.Function):
         have_tail = bool(ctx.tail)
         first = 1 if have_tail else 0  # the first segment to recompute (in reverse order)
         # one buffer per segment to recompute, at most two, taken in turn
-        bufs = [[torch.empty(shape, dtype=torch.float64, device=dev) for _ in range(K - 1)]
+        bufs = [list(torch.empty((K - 1,) + shape, dtype=torch.float64, device=dev))
                 for _ in range(min(2, len(order) - first))]
         ready = [None] * len(order)
         free = [None, None]
