@@ -38,12 +38,6 @@ namespace claw {
 constexpr int kLanes = 64;
 constexpr int kOwn = 60;  // owned columns per strip
 constexpr int kWPB = 4;   // independent wavefronts per workgroup, at least
-// Shallow-water steady rows per segment from which issue priority follows progress (shorter
-// segments ran 0.5-2% slower with it on MI355X: 2048^2 and below)
-constexpr int kPrioRows = 64;
-// the same for the Euler kernels (about twice the work per row): marched rows per segment
-constexpr int kPrioRowsEuler = 16;
-
 static thread_local std::string g_err;
 static int fail(int code, const std::string& msg) {
   g_err = msg;
@@ -460,12 +454,46 @@ __device__ __forceinline__ void publish_max(claw2d_ctrl* c, const ItemMax& m, bo
   if (m.bad) atomicOr(&c->status, (int)CLAW_STATUS_BAD_STATE);
 }
 
+// Issue priority from relative progress.  Two to four wavefronts of a workgroup share a SIMD, with
+// equal work, and the arbiter favours the oldest: at 2048^2 (FP64 shallow water) one of each pair
+// finished after 50 us and the other ran the last 27 us alone, where a row takes 1.1 us against 0.91
+// of a pair.  So every wavefront keeps its rows to go in LDS, compares them now and then with those of
+// the wavefronts that share its SIMD (they are dealt to the 4 SIMDs in turn), and issues at a lower
+// priority the more of them have more to do.  Issue order only: no result bit changes.  2048^2: FP64
+// 85 -> 81 us, split 68 -> 64, FP32 56.5 -> 52.7; bathymetry FP32 3000 x 2000 74 -> 68; FP32 Euler 1501 x
+// 1207 51.5 -> 47.9; 4096^2 (where the priority had followed the quarters of a segment) 178 -> 177
+// FP32, 310 -> 308 FP64.
+struct Progress {
+  int* rows = nullptr;     // LDS, per wavefront of the workgroup: minus its rows to go, INT_MAX: none
+  int slot = 0, n = 0;     // this wavefront's entry, and the number of entries
+  int seen = 0, mine = 0;  // the entry this lane looked up last, and this wavefront's own then
+  __device__ __forceinline__ bool on() const { return n > 4; }
+  __device__ __forceinline__ void look(int lane) {
+    const int k = (slot & 3) + 4 * lane;
+    seen = __hip_atomic_load(&rows[k < n ? k : slot], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+  }
+  __device__ __forceinline__ void put(int row) {
+    __hip_atomic_store(&rows[slot], row, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+  }
+  // r: minus the rows to go.  Acts on the entries looked up at the last call (the rows between hid
+  // their latency).
+  __device__ __forceinline__ void at(int r, int lane) {
+    const int behind = __builtin_popcountll(__builtin_amdgcn_ballot_w64(seen < mine));
+    if (behind == 0) __builtin_amdgcn_s_setprio(2);
+    else if (behind == 1) __builtin_amdgcn_s_setprio(1);
+    else __builtin_amdgcn_s_setprio(0);
+    mine = r;
+    put(r);
+    look(lane);  // (its own entry is never below mine)
+  }
+};
+
 template <class T, class P, int LIM, bool SPLIT = false, int TWC = -1, bool PAD = false, int SWEEP = 0,
           bool CAPA = false>
 __device__ __forceinline__ ItemMax march_item(const StepArgs<T, P>& a, const T* __restrict__ qin,
                                            T* __restrict__ qout, const int mx, const int my,
                                            const int x0, const int y0, const int y1, const double dt,
-                                           const double dx, const double dy) {
+                                           const double dx, const double dy, const Progress pg = Progress{}) {
   static_assert(SWEEP == 0 || (SPLIT && PAD), "single sweeps run on the padded split path");
   static_assert(!(CAPA && PAD), "the capacity form runs on the index-mapped (unpadded) path");
   constexpr bool DPP = kDppShift<T, P>;
@@ -860,26 +888,9 @@ __device__ __forceinline__ ItemMax march_item(const StepArgs<T, P>& a, const T* 
     int R = rlo;
     const int ys = min(y1, my - 1);  // first row past the steady ones
     for (; R < y0 + 2 && R <= rhi; ++R) row(R, std::false_type{});
-    // Issue priority from progress (segments of at least kPrioRows steady rows): 3 over the first
-    // quarter of the steady rows, then 2, 1 and 0.  The wavefronts that share a SIMD start
-    // together with equal work, and the arbiter otherwise favours the older one: it finishes
-    // early and the others run their last stretch with fewer wavefronts per SIMD.  With the
-    // priority falling as a wavefront advances, the one behind is issued first, and they finish
-    // closer together.  Issue order only: no result bit changes.  (For FP32 it measured slower
-    // while every wavefront still sent its own device-scope atomics at its end: finishing together
-    // queued them; with one set per workgroup it is 7% faster at 4096^2, 10% at 8192^2.)
-    const bool prio = ys - R >= kPrioRows;
-    const int pq = max((ys - R) >> 2, 1);
-    int Rq = prio ? R + pq : INT_MAX, pl = 3;  // next row at which the priority steps down
-    if (prio) __builtin_amdgcn_s_setprio(3);
+    Progress prog = pg;
     auto prio_at = [&](int r) {
-      if (r >= Rq) {
-        Rq += pq;
-        --pl;
-        if (pl == 2) __builtin_amdgcn_s_setprio(2);
-        else if (pl == 1) __builtin_amdgcn_s_setprio(1);
-        else __builtin_amdgcn_s_setprio(0);
-      }
+      if (prog.on()) prog.at(r - rhi, lane);
     };
     if constexpr (sizeof(T) == 8 && NEQ == 3 && (SPLIT || !P::FWAVE)) {
       // two steady rows per iteration: the rolling window's registers are renamed, not copied (33
@@ -895,17 +906,22 @@ __device__ __forceinline__ ItemMax march_item(const StepArgs<T, P>& a, const T* 
       prio_at(R);
       row(R, std::true_type{});
     }
-    if (prio) __builtin_amdgcn_s_setprio(0);
+    if (prog.on()) {
+      prog.put(INT_MAX);
+      __builtin_amdgcn_s_setprio(0);
+    }
     for (; R <= rhi; ++R) row(R, std::false_type{});
   } else {
-    // Issue priority from progress, as above, over every marched row of an Euler segment (2048^2
-    // on MI355X: FP64 -5%, FP32 -10%)
-    const bool prio = NEQ == 4 && rhi - rlo >= kPrioRowsEuler;
+    // FP64 unsplit Euler has no register for the look-ups (2048^2 132 -> 148 us with them) and lowers
+    // the priority from 3 to 0 over the quarters of its segment instead, which bounds a lead.
+    constexpr bool kQuarters = NEQ == 4 && sizeof(T) == 8 && !SPLIT;
+    Progress prog = pg;
+    const bool prio = kQuarters && rhi - rlo >= 16;
     const int pq = max((rhi + 1 - rlo) >> 2, 1);
     int Rq = prio ? rlo + pq : INT_MAX, pl = 3;
     if (prio) __builtin_amdgcn_s_setprio(3);
     for (int R = rlo; R <= rhi; ++R) {
-      if constexpr (NEQ == 4) {
+      if constexpr (kQuarters) {
         if (R >= Rq) {
           Rq += pq;
           --pl;
@@ -913,10 +929,13 @@ __device__ __forceinline__ ItemMax march_item(const StepArgs<T, P>& a, const T* 
           else if (pl == 1) __builtin_amdgcn_s_setprio(1);
           else __builtin_amdgcn_s_setprio(0);
         }
+      } else if (prog.on()) {
+        prog.at(R - rhi, lane);
       }
       row(R, std::false_type{});
     }
-    if (prio) __builtin_amdgcn_s_setprio(0);
+    if (!kQuarters && prog.on()) prog.put(INT_MAX);
+    if (prio || prog.on()) __builtin_amdgcn_s_setprio(0);
   }
 
   // Wave-uniform epilogue: no lane-divergent branch (a lane-0-only branch here lets the compiler
@@ -1029,11 +1048,12 @@ __device__ __forceinline__ void control_one(claw2d_ctrl* c, double dx, double dy
 #endif
 // Wavefronts per workgroup a single-grid kernel is built for: those one CU holds at the kernel's
 // registers (FP64 2 per SIMD, its specialised split kernels 3; FP32 4, Euler 3), so that a CU can
-// run one workgroup, which sends one set of atomics.  FP64 Euler keeps 4: 8 gained nothing there.
+// run one workgroup, which sends one set of atomics.  FP64 unsplit Euler keeps 4: 8 gained
+// nothing there.
 // METHOD: the method is fixed at compile time.
 template <class T, class P, bool SPLIT, bool METHOD>
 constexpr int kMaxWPB =
-    sizeof(T) == 8 ? (P::NEQ == 4 ? 4 : (SPLIT && METHOD ? 12 : 8)) : (P::NEQ == 3 ? 16 : 12);
+    sizeof(T) == 8 ? (P::NEQ == 4 && !SPLIT ? 4 : (P::NEQ == 3 && SPLIT && METHOD ? 12 : 8)) : (P::NEQ == 3 ? 16 : 12);
 
 template <class T> struct MinWaves {
   static constexpr int value = sizeof(T) == 8 ? CLAW_MIN_WAVES_F64 : CLAW_MIN_WAVES_F32;
@@ -1048,7 +1068,8 @@ step2_fused(StepArgs<T, P> a) {
   // had queued at the end of the step: removing them made FP32 shallow water at 4096^2 17%
   // faster on MI355X, and a workgroup of 4 wavefronts sends a quarter of them.
   __shared__ unsigned long long wg_smax[2];
-  __shared__ int wg_bad, wg_arrived;
+  __shared__ int wg_bad, wg_arrived, wg_rows[kMaxWPB<T, P, SPLIT, (LIM > 0)>];
+  if ((int)threadIdx.x < kMaxWPB<T, P, SPLIT, (LIM > 0)>) wg_rows[threadIdx.x] = INT_MAX;
   if (threadIdx.x == 0) {
     wg_smax[0] = wg_smax[1] = 0ull;
     wg_bad = 0;
@@ -1070,8 +1091,12 @@ step2_fused(StepArgs<T, P> a) {
   const int strip = wave % a.nstrips, seg = wave / a.nstrips;
   const int x0 = strip * kOwn, y0 = seg * a.seg_h;
   const int y1 = min(y0 + a.seg_h, a.my);
+  Progress pg;
+  pg.rows = wg_rows;
+  pg.slot = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  pg.n = a.wpb;
   const ItemMax m = march_item<T, P, LIM, SPLIT, TWC, PAD, SWEEP, CAPA>(a, qin, qout, a.mx, a.my, x0, y0, y1,
-                                                                       dt, a.dx, a.dy);
+                                                                       dt, a.dx, a.dy, pg);
   const int lane = threadIdx.x & 63;
   atomicMax(&wg_smax[0], (unsigned long long)__double_as_longlong(m.sx));
   atomicMax(&wg_smax[1], (unsigned long long)__double_as_longlong(m.sy));
@@ -1122,6 +1147,7 @@ struct BatchDev {
   int* counter;
   int ngrids;
   int total_items;
+  int wpb;  // wavefronts per workgroup
 };
 
 // The last grid whose item0 <= item (item0 ascends from 0): 64 grids are probed at once, one per lane.
@@ -1139,11 +1165,18 @@ __device__ __forceinline__ int grid_of_item(const BatchDev& b, int item) {
 }
 
 template <class T, class P, int LIM, int TWC>
-__global__ void __launch_bounds__(kLanes* kWPB) __attribute__((amdgpu_waves_per_eu(MinWaves<T>::value)))
+__global__ void __launch_bounds__(kLanes*(kMaxWPB<T, P, false, true>)) __attribute__((amdgpu_waves_per_eu(MinWaves<T>::value)))
 batch_step(StepArgs<T, P> a, BatchDev b) {
   const int lane = threadIdx.x & 63;
-  const int first = (int)gridDim.x * kWPB;  // items taken by number
-  int item = __builtin_amdgcn_readfirstlane(xcd_remap(blockIdx.x, gridDim.x) * kWPB + (threadIdx.x >> 6));
+  __shared__ int wg_rows[kMaxWPB<T, P, false, true>];
+  if ((int)threadIdx.x < kMaxWPB<T, P, false, true>) wg_rows[threadIdx.x] = INT_MAX;
+  __syncthreads();  // before any wavefront of the workgroup leaves
+  Progress pg;
+  pg.rows = wg_rows;
+  pg.slot = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  pg.n = b.wpb;
+  const int first = (int)gridDim.x * b.wpb;  // items taken by number
+  int item = __builtin_amdgcn_readfirstlane(xcd_remap(blockIdx.x, gridDim.x) * b.wpb + pg.slot);
   // no lane-divergent region sits inside this loop (every lane takes part in the tickets: lane 0 adds
   // 1, the others 0; every lane runs the controller, all with the same values)
   while (item < b.total_items) {
@@ -1158,7 +1191,8 @@ batch_step(StepArgs<T, P> a, BatchDev b) {
       const int strip = local % G.nstrips, seg = local / G.nstrips;
       const int x0 = strip * kOwn, y0 = seg * G.seg_h;
       const int y1 = min(y0 + G.seg_h, G.my);
-      publish_max(c, march_item<T, P, LIM, false, TWC>(a, qin, qout, G.mx, G.my, x0, y0, y1, dt, G.dx, G.dy), false);
+      publish_max(c, march_item<T, P, LIM, false, TWC>(a, qin, qout, G.mx, G.my, x0, y0, y1, dt, G.dx, G.dy, pg),
+                  false);
       // the maxima are performed before the arrival (see step2_fused)
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
       const int arrived = __builtin_amdgcn_readfirstlane(atomicAdd(&c->arrive, lane == 0 ? 1 : 0));
@@ -1345,9 +1379,9 @@ static int launch_wpb(const claw2d_desc* d) { return d->wg_waves > 0 ? d->wg_wav
 // in one workgroup each, up to what the kernel is built for.  Fewer, larger workgroups send fewer
 // atomics (beside the lookup in publish_max: shallow water 2048^2 FP32 70.8 -> 69.2 us, bathymetry
 // FP32 69.9 -> 66.2 us, FP64 minmod 97.3 -> 94.8 us).
-static int fit_wpb(const claw2d_desc* d, long items, int most) {
+static int fit_wpb(long items, int most) {
   const long cus = device_simds() / 4;
-  if (launch_wpb(d) < kWPB || cus <= 0) return launch_wpb(d);
+  if (cus <= 0) return kWPB;
   return (int)std::min<long>(most, std::max<long>(kWPB, (items + cus - 1) / cus));
 }
 // occupancy cache index of a wavefronts-per-workgroup count 1, 2 or 4
@@ -1571,7 +1605,9 @@ static int launch_step(const claw2d_desc* d, const typename P::Par& par, void* q
   const int waves = a.nstrips * a.nsegs;
   a.total_waves = waves;
   const int wpb = a.wpb =
-      fit_wpb(d, waves, SPLIT && slot < 2 ? kMaxWPB<T, P, SPLIT, true> : kMaxWPB<T, P, SPLIT, false>);
+      launch_wpb(d) < kWPB
+          ? launch_wpb(d)
+          : fit_wpb(waves, SPLIT && slot < 2 ? kMaxWPB<T, P, SPLIT, true> : kMaxWPB<T, P, SPLIT, false>);
   const int blocks = (waves + wpb - 1) / wpb;
   void* args[] = {&a};
   const hipError_t e = hipLaunchKernel(kern, dim3(blocks), dim3(kLanes * wpb), args, 0, s);
@@ -1698,9 +1734,10 @@ static int launch_batch(const claw2d_desc* d, const typename P::Par& par, const 
   b.total_items = total_items;
   const long res = resident > 0 ? resident : 4096;
   const long waves = std::min<long>(total_items, res);
-  const int blocks = (int)((waves + kWPB - 1) / kWPB);
+  const int wpb = b.wpb = fit_wpb(waves, kMaxWPB<T, P, false, true>);
+  const int blocks = (int)((waves + wpb - 1) / wpb);
   void* args[] = {&a, &b};
-  const hipError_t e = hipLaunchKernel(kern, dim3(blocks), dim3(kLanes * kWPB), args, 0, s);
+  const hipError_t e = hipLaunchKernel(kern, dim3(blocks), dim3(kLanes * wpb), args, 0, s);
   return e == hipSuccess ? 0 : hip_fail(e, "batch_step launch");
 }
 
