@@ -38,6 +38,9 @@ SOURCES = [
     ("claw2d_euler64.hip", ["-mllvm", "-amdgpu-sched-strategy=max-ilp"]),
     # FP32 Euler (MC, transverse_waves 2): -1.1%
     ("claw2d_euler32.hip", ["-mllvm", "-amdgpu-sched-strategy=max-ilp"]),
+    # superbee, van Leer and transverse_waves 0, the default scheduler
+    ("claw2d_lim64.hip", []),
+    ("claw2d_lim32.hip", []),
 ]
 
 

@@ -834,6 +834,10 @@ __device__ __forceinline__ ItemMax march_item(const StepArgs<T, P>& a, const T* 
 #pragma unroll
         for (int m = 0; m < NEQ; ++m) {
           const T X = RX[m] + from_right<DPP, T, DPPZ>(LX[m]);
+          if constexpr (TWC == 0) {  // no transverse shares
+            acc2[m] += X;
+            continue;
+          }
           const T G1 = RG1[m] + from_right<DPP, T, DPPZ>(LG1[m]);
           const T G2 = RG2[m] + from_right<DPP, T, DPPZ>(LG2[m]);
           acc1[m] -= G1;
@@ -1341,6 +1345,32 @@ extern template __global__ void step2_fused<float, SweP<float>, 4, false, 2, fal
 CLAW_EULER64_KERNELS(CLAW_EULER64_EXTERN)
 extern template __global__ void step2_fused<float, EulerP<float>, 4, false, 2, false, 0, false>(
     StepArgs<float, EulerP<float>>);
+// Superbee (2) and van Leer (3), the method fixed at compile time like MC's and minmod's: in units of
+// their own for the build's sake (claw2d_lim64.hip, claw2d_lim32.hip).  Against the general kernel:
+// van Leer FP64 4096^2 351 -> 324 us, split 2048^2 86 -> 73.5, 1023 x 777 37.2 -> 34.2, FP32 2048^2
+// 63.5 -> 57.5; superbee 87 -> 78.7, Euler 1800 x 1700 105 -> 95, bathymetry split 2048^2 80 -> 68.
+// transverse_waves 0: MC FP64 2048^2 78 -> 68 us, FP32 54 -> 44, Euler 1800 x 1700 93 -> 77.
+#define CLAW_LIMITER_KERNELS(K, T)                                                              \
+  K(T, SweP<T>, 2, false, 2) K(T, SweP<T>, 3, false, 2) K(T, SweP<T>, 2, false, 1) K(T, SweP<T>, 3, false, 1) \
+  K(T, SweP<T>, 2, true, 0) K(T, SweP<T>, 3, true, 0)                                           \
+  K(T, SweBathyP<T>, 2, false, 2) K(T, SweBathyP<T>, 3, false, 2) K(T, SweBathyP<T>, 2, false, 1) \
+  K(T, SweBathyP<T>, 3, false, 1) K(T, SweBathyP<T>, 2, true, 0) K(T, SweBathyP<T>, 3, true, 0) \
+  K(T, EulerP<T>, 2, false, 2) K(T, EulerP<T>, 3, false, 2) K(T, EulerP<T>, 2, false, 1)        \
+  K(T, EulerP<T>, 3, false, 1) K(T, EulerP<T>, 2, true, 0) K(T, EulerP<T>, 3, true, 0)
+// transverse_waves 0, every limiter
+#define CLAW_NO_TRANSVERSE_KERNELS(K, T)                                                            \
+  K(T, SweP<T>, 1, false, 0) K(T, SweP<T>, 2, false, 0) K(T, SweP<T>, 3, false, 0) K(T, SweP<T>, 4, false, 0) \
+  K(T, SweBathyP<T>, 1, false, 0) K(T, SweBathyP<T>, 2, false, 0) K(T, SweBathyP<T>, 3, false, 0)   \
+  K(T, SweBathyP<T>, 4, false, 0) K(T, EulerP<T>, 1, false, 0) K(T, EulerP<T>, 2, false, 0)         \
+  K(T, EulerP<T>, 3, false, 0) K(T, EulerP<T>, 4, false, 0)
+#define CLAW_LIMITER_EXTERN(T, P, LIM, SPLIT, TWC) \
+  extern template __global__ void step2_fused<T, P, LIM, SPLIT, TWC, false, 0, false>(StepArgs<T, P>);
+#define CLAW_LIMITER_DEFINE(T, P, LIM, SPLIT, TWC) \
+  template __global__ void step2_fused<T, P, LIM, SPLIT, TWC, false, 0, false>(StepArgs<T, P>);
+CLAW_LIMITER_KERNELS(CLAW_LIMITER_EXTERN, double)
+CLAW_LIMITER_KERNELS(CLAW_LIMITER_EXTERN, float)
+CLAW_NO_TRANSVERSE_KERNELS(CLAW_LIMITER_EXTERN, double)
+CLAW_NO_TRANSVERSE_KERNELS(CLAW_LIMITER_EXTERN, float)
 
 #ifndef CLAW_KERNEL_UNIT
 // ------------------------------------------------------------------------------------------
@@ -1395,10 +1425,10 @@ static const double* row_times(const claw2d_desc* d, bool split) {
   static const double kRel64Split[4] = {1.0, 1.5, 2.15, 2.8}, kRel32[4] = {1.0, 1.22, 1.55, 2.0};
   bool same = true;
   for (int p = 1; p < d->num_waves; ++p) same = same && d->mthlim[p] == d->mthlim[0];
-  const bool own = same && (d->mthlim[0] == 1 || d->mthlim[0] == 4);  // a limiter with kernels of its own
+  const bool own = same && d->mthlim[0] >= 1 && d->mthlim[0] <= 4 && d->order == 2;  // kernels of its own
   if (d->dtype != CLAW_FP64) return kRel32;
   if (d->solver == CLAW_SOLVER_EULER_4WAVE || !own) return kRel64Long;
-  return split ? kRel64Split : kRel64;
+  return split || d->transverse_waves == 0 ? kRel64Split : kRel64;
 }
 
 // Rows per marching segment.  A wavefront's run time is proportional to its rows (4 of them halo
@@ -1543,31 +1573,36 @@ template <class T> static typename EulerP<T>::Par euler_par(const claw2d_desc* d
   return p;
 }
 
-// Kernel variant for a method: a uniform MC or minmod limiter at order 2 with the transverse
-// mode fixed at compile time (split: none; unsplit: 1 or 2), else the general kernel (per-wave
-// limiter ids, order and transverse_waves read at run time).  slot indexes the occupancy cache.
+// Kernel variant for a method: one limiter of minmod, superbee, van Leer and MC for all waves at
+// order 2 with the transverse mode fixed at compile time (split: none; unsplit: 0, 1 or 2), else the
+// general kernel (per-wave limiter ids, order and transverse_waves read at run time).  slot indexes
+// the occupancy cache.
+template <class T, class P, bool SPLIT, int TWC> static const void* limiter_kernel(int lim) {
+  switch (lim) {
+    case 1: return (const void*)step2_fused<T, P, 1, SPLIT, TWC>;
+    case 2: return (const void*)step2_fused<T, P, 2, SPLIT, TWC>;
+    case 3: return (const void*)step2_fused<T, P, 3, SPLIT, TWC>;
+    default: return (const void*)step2_fused<T, P, 4, SPLIT, TWC>;
+  }
+}
+constexpr int kSlotGeneral = 12, kSlotPad = 13, kSlotCapa = 14, kSlots = 15;
 template <class T, class P, bool SPLIT>
 static const void* step_kernel(const claw2d_desc* d, int* slot) {
   bool same = true;
   for (int p = 1; p < P::NW; ++p) same = same && d->mthlim[p] == d->mthlim[0];
   const int lim = same ? d->mthlim[0] : -1;
-  if ((lim == 4 || lim == 1) && d->order == 2) {
-    const bool mc = lim == 4;
+  if (lim >= 1 && lim <= 4 && d->order == 2) {
     if constexpr (SPLIT) {
-      *slot = mc ? 0 : 1;
-      return mc ? (const void*)step2_fused<T, P, 4, true, 0> : (const void*)step2_fused<T, P, 1, true, 0>;
+      *slot = lim - 1;
+      return limiter_kernel<T, P, true, 0>(lim);
     } else {
-      if (d->transverse_waves == 2) {
-        *slot = mc ? 0 : 1;
-        return mc ? (const void*)step2_fused<T, P, 4, false, 2> : (const void*)step2_fused<T, P, 1, false, 2>;
-      }
-      if (d->transverse_waves == 1) {
-        *slot = mc ? 2 : 3;
-        return mc ? (const void*)step2_fused<T, P, 4, false, 1> : (const void*)step2_fused<T, P, 1, false, 1>;
-      }
+      *slot = 4 * d->transverse_waves + lim - 1;
+      if (d->transverse_waves == 2) return limiter_kernel<T, P, false, 2>(lim);
+      if (d->transverse_waves == 1) return limiter_kernel<T, P, false, 1>(lim);
+      return limiter_kernel<T, P, false, 0>(lim);
     }
   }
-  *slot = 4;
+  *slot = kSlotGeneral;
   return (const void*)step2_fused<T, P, 0, SPLIT, -1>;
 }
 
@@ -1575,18 +1610,22 @@ template <class T, class P, bool SPLIT>
 static int launch_step(const claw2d_desc* d, const typename P::Par& par, void* q0, void* q1,
                        const void* aux, claw2d_ctrl* ctrl, int use_ctrl, double dt, hipStream_t s,
                        bool pad = false) {
-  int slot = 5;
+  int slot = kSlotPad;
   const void* kern = (const void*)step2_fused<T, P, 0, false, -1, true>;
   if (d->mcapa > 0) {
-    slot = 6;  // the capacity form runs the general kernel
+    slot = kSlotCapa;  // the capacity form runs the general kernel
     kern = (const void*)step2_fused<T, P, 0, SPLIT, -1, false, 0, true>;
   } else if (!pad || SPLIT) {
     kern = step_kernel<T, P, SPLIT>(d, &slot);
   }
-  static thread_local long cached[7][3] = {{-1, -1, -1}, {-1, -1, -1}, {-1, -1, -1}, {-1, -1, -1},
-                                           {-1, -1, -1}, {-1, -1, -1}, {-1, -1, -1}};
+  static thread_local long cached[kSlots][3];  // 0: not queried yet (no kernel holds 0)
   long& res = cached[slot][wpb_index(launch_wpb(d))];
-  if (res < 0) res = resident_waves(kern, launch_wpb(d));
+  // the most wavefronts a workgroup of this launch may hold: the occupancy counts such workgroups (a
+  // kernel that fits 12 wavefronts on a CU holds one workgroup of 8: cut for 12, half of them would
+  // run in a second round)
+  const int most = slot < kSlotGeneral ? kMaxWPB<T, P, SPLIT, true> : kMaxWPB<T, P, SPLIT, false>;
+  const int packing = launch_wpb(d) < kWPB ? launch_wpb(d) : most;
+  if (res <= 0) res = resident_waves(kern, packing);
   StepArgs<T, P> a;
   fill_args(a, d, res, SPLIT);
   a.q0 = (T*)q0;
@@ -1604,10 +1643,7 @@ static int launch_step(const claw2d_desc* d, const typename P::Par& par, void* q
   if (d->mcapa > 0) a.capa = (const T*)aux + (size_t)(d->mcapa - 1) * (size_t)d->mx * (size_t)d->my;
   const int waves = a.nstrips * a.nsegs;
   a.total_waves = waves;
-  const int wpb = a.wpb =
-      launch_wpb(d) < kWPB
-          ? launch_wpb(d)
-          : fit_wpb(waves, SPLIT && slot < 2 ? kMaxWPB<T, P, SPLIT, true> : kMaxWPB<T, P, SPLIT, false>);
+  const int wpb = a.wpb = launch_wpb(d) < kWPB ? launch_wpb(d) : fit_wpb(waves, most);
   const int blocks = (waves + wpb - 1) / wpb;
   void* args[] = {&a};
   const hipError_t e = hipLaunchKernel(kern, dim3(blocks), dim3(kLanes * wpb), args, 0, s);
