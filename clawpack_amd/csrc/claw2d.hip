@@ -1161,7 +1161,7 @@ __device__ __forceinline__ int grid_of_item(const BatchDev& b, int item) {
   while (n > 1) {
     const int stride = (n + 63) >> 6, k = lane * stride;
     const unsigned long long le = lanes(k < n && b.grids[lo + (k < n ? k : 0)].item0 <= item);
-    const int j = 63 - __builtin_clzll(le);  // lane 0 always holds; lanes that hold are 0 .. j
+    const int j = 63 - __builtin_clzll(le | 1ull);  // lanes that hold are 0 .. j
     lo += j * stride;
     n = min(stride, n - j * stride);
   }
@@ -1800,7 +1800,7 @@ static int batch_rows(const claw2d_desc* d, const claw2d_batch_grid* grids, int 
   const long most = std::min(4L, slots / simds);
   int best_h = 64;
   double best = 1e300;
-  for (int h = 2; h <= std::min(most_rows, 256); ++h) {
+  for (int h = 2; h <= std::min(most_rows, 256); h += std::max(1, h / 16)) {
     long items = 0;
     double rows = 0.0;  // with the 6 rows' worth of a segment's own cost
     int longest = 0;
